@@ -1,7 +1,7 @@
 // The `feather_ops` torch library and the `feather_ops._C` Python module (reference: csrc/extension.cpp:1-23
 // plus the op registration of csrc/hip_kernel.cu:716-846). Host code only: it validates the tensors,
 // takes the current stream of a's device, and calls the C ABI of libfeather_ops_gfx950.so
-// (include/feather_ops.h). Built against torch's stable ABI, like the reference.
+// (include/feather_ops.h, and feather_internal.h for what only it calls). Built against torch's stable ABI, like the reference.
 #include <Python.h>
 
 #include <torch/csrc/stable/accelerator.h>
@@ -13,7 +13,7 @@
 #include <cstdint>
 #include <optional>
 
-#include "feather_ops.h"
+#include "feather_internal.h"
 
 namespace {
 
@@ -243,6 +243,65 @@ void prepack_b(const Tensor& b, Tensor& out) {
     STD_TORCH_CHECK(err == hipSuccess, "prepack_b kernel launch failed: ", hipGetErrorString(err));
 }
 
+// feather_ops::linear_backward: feather_linear_backward on tensors (grad [M, N], b_prepacked [K_pad/16, N, 16], scale of
+// one or N elements; grad_x [M, K] and grad_bias [N] in grad's dtype, each optional). split_workspace: as
+// scaled_mm_splitk's, ignored for splits = 1. workspace: uint8, any content.
+void linear_backward(const Tensor& grad, const Tensor& b_prepacked, const Tensor& scale,
+                     std::optional<Tensor> grad_x, std::optional<Tensor> grad_bias, Tensor& split_workspace,
+                     Tensor& workspace, const int64_t K, const int64_t splits, const int64_t block_warps_m,
+                     const int64_t block_warps_n, const int64_t unroll_k, const int64_t repeat_m,
+                     const int64_t repeat_n, const bool prefetch) {
+    STD_TORCH_CHECK(grad.is_cuda() && b_prepacked.is_cuda() && scale.is_cuda() && workspace.is_cuda() &&
+                        split_workspace.is_cuda(),
+                    "grad, b_prepacked, scale and the workspaces must be CUDA tensors");
+    const auto device_index = grad.get_device_index();
+    STD_TORCH_CHECK(b_prepacked.get_device_index() == device_index && scale.get_device_index() == device_index &&
+                        workspace.get_device_index() == device_index &&
+                        split_workspace.get_device_index() == device_index,
+                    "grad, b_prepacked, scale and the workspaces must be on one device");
+    const auto type = grad.scalar_type();
+    STD_TORCH_CHECK(type == ST::Half || type == ST::BFloat16, "grad must be float16 or bfloat16");
+    const auto b_type = b_prepacked.scalar_type();
+    STD_TORCH_CHECK(b_type == ST::Float8_e4m3fn || b_type == ST::Float8_e5m2,
+                    "b_prepacked must be float8_e4m3fn or float8_e5m2");
+    STD_TORCH_CHECK(grad.dim() == 2 && b_prepacked.dim() == 3, "grad must be 2-D and b_prepacked 3-D");
+    const int64_t M = grad.size(0);
+    const int64_t N = grad.size(1);
+    STD_TORCH_CHECK(M >= 1 && N >= 8 && N % 8 == 0 && K >= 16 && K % 16 == 0,
+                    "linear_backward needs M >= 1, N a multiple of 8 and K of 16");
+    STD_TORCH_CHECK(b_prepacked.size(0) >= K / 16 && b_prepacked.size(1) == N && b_prepacked.size(2) == 16,
+                    "b_prepacked must be [K_pad/16, N, 16]");
+    STD_TORCH_CHECK(grad.is_contiguous() && b_prepacked.is_contiguous(), "grad and b_prepacked must be contiguous");
+    STD_TORCH_CHECK(scale.scalar_type() == ST::Float && (scale.numel() == 1 || scale.numel() == N) &&
+                        (scale.numel() == 1 || scale.is_contiguous()),
+                    "scale must be float32 with one element or N contiguous ones");
+    if (grad_x.has_value()) {
+        STD_TORCH_CHECK(grad_x->is_cuda() && grad_x->get_device_index() == device_index &&
+                            grad_x->scalar_type() == type && grad_x->dim() == 2 && grad_x->size(0) == M &&
+                            grad_x->size(1) == K && grad_x->is_contiguous(),
+                        "grad_x must be a contiguous [M, K] tensor of grad's dtype on its device");
+    }
+    if (grad_bias.has_value()) {
+        STD_TORCH_CHECK(grad_bias->is_cuda() && grad_bias->get_device_index() == device_index &&
+                            grad_bias->scalar_type() == type && grad_bias->numel() == N && grad_bias->is_contiguous(),
+                        "grad_bias must be a contiguous tensor of N elements of grad's dtype on its device");
+    }
+    STD_TORCH_CHECK(workspace.scalar_type() == ST::Byte && workspace.is_contiguous() &&
+                        split_workspace.scalar_type() == ST::Byte && split_workspace.is_contiguous(),
+                    "the workspaces must be contiguous uint8 tensors");
+    torch::stable::accelerator::DeviceGuard guard(device_index);
+    const bool launched = feather_linear_backward(
+        static_cast<const uint16_t*>(grad.const_data_ptr()), static_cast<const uint8_t*>(b_prepacked.const_data_ptr()),
+        static_cast<const float*>(scale.const_data_ptr()),
+        grad_x.has_value() ? static_cast<uint16_t*>(grad_x->mutable_data_ptr()) : nullptr,
+        grad_bias.has_value() ? static_cast<uint16_t*>(grad_bias->mutable_data_ptr()) : nullptr, M, N, K,
+        scale.numel() != 1, b_type == ST::Float8_e5m2, type == ST::BFloat16, static_cast<int>(block_warps_m),
+        static_cast<int>(block_warps_n), static_cast<int>(unroll_k), static_cast<int>(repeat_m),
+        static_cast<int>(repeat_n), prefetch, static_cast<int>(splits), split_workspace.mutable_data_ptr(),
+        split_workspace.numel(), workspace.mutable_data_ptr(), workspace.numel(), current_stream(device_index));
+    check_launch(launched, "linear_backward");
+}
+
 }  // namespace
 
 STABLE_TORCH_LIBRARY(feather_ops, m) {
@@ -256,6 +315,10 @@ STABLE_TORCH_LIBRARY(feather_ops, m) {
     m.def("bf16_to_fp16(Tensor x, Tensor(a!) out) -> ()");
     m.def("widen_bf16(Tensor x, Tensor(a!) out) -> ()");
     m.def("prepack_b(Tensor b, Tensor(a!) out) -> ()");
+    m.def(
+        "linear_backward(Tensor grad, Tensor b_prepacked, Tensor scale, Tensor(a!)? grad_x, Tensor(b!)? grad_bias, "
+        "Tensor(c!) split_workspace, Tensor(d!) workspace, int K, int splits, int block_warps_m, int block_warps_n, "
+        "int unroll_k, int repeat_m, int repeat_n, bool prefetch) -> ()");
 }
 
 STABLE_TORCH_LIBRARY_IMPL(feather_ops, CUDA, m) {
@@ -264,6 +327,7 @@ STABLE_TORCH_LIBRARY_IMPL(feather_ops, CUDA, m) {
     m.impl("bf16_to_fp16", TORCH_BOX(&bf16_to_fp16));
     m.impl("widen_bf16", TORCH_BOX(&widen_bf16));
     m.impl("prepack_b", TORCH_BOX(&prepack_b));
+    m.impl("linear_backward", TORCH_BOX(&linear_backward));
 }
 
 extern "C" PyObject* PyInit__C(void) {

@@ -1,0 +1,359 @@
+// Gradients of y = (x @ W^T) * scale + bias for a frozen prepacked fp8 weight W:
+//   grad_x[m, k]  = sum_n grad[m, n] * scale[n] * W[n, k]        grad_bias[n] = sum_m grad[m, n]
+// grad_x is the forward's own matmul on the transposed weight: the prepacked [K/16][N][16] becomes [N/16][K][16]
+// (one pass over the weight, here), and the ring, wide and streaming kernels contract over N.
+//
+// The products are those of fp32 arithmetic, on the 16-bit MFMAs: an fp8 code is exact in fp16 and bf16, so a
+// 16-bit gradient times a code is exact in the fp32 accumulator. A per-tensor scale goes into the decode (its
+// power of two) and the epilogue. A per-column scale sits inside the sum: grad * scale is formed in fp32 and split
+// into three bf16 terms that sum to it exactly (split_columns_kernel), and the matmul runs over the three side by
+// side, a contraction three times as long over three copies of the weight.
+//
+// Measured, forward and backward of 4096 rows through 3072 -> 12288 in bf16, one scale: 2732 us with torch's fp32
+// operations (1.9 ms its fp32 matmul, 0.27 ms the column sums, 0.2 ms dequantizing the weight), 435 us here: the
+// matmul's 309 GFLOP take 215-238 us (1.3-1.4 PFLOP/s, the rate of the forward's). 1000 rows through 2560 -> 5120 in
+// fp16 with per-column scales: 322 us, 158 us here (the three-term matmul 78 us, 1.0 PFLOP/s).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+
+#include "feather_internal.h"
+#include "scaled_mm_kernels.h"
+#include "scaled_mm_launch.h"
+
+namespace feather {
+namespace {
+
+constexpr int kThreads = 256;
+
+// ---- weight transpose ----------------------------------------------------------------------------------------
+//
+// b [K/16][N][16] -> out [copies][N16][K][16], N16 = ceil(N / 16): out[c][n / 16][k][n % 16] = b[k / 16][n][k % 16],
+// zero for n >= N. Copies after the first (e5m2) hold zero for an infinite code: they meet the small terms of the split
+// gradient, and a zero term times inf would add NaN to the first copy's inf. A workgroup takes 8 chunks of k by 128 columns n (16 KiB): 2 KiB runs in, 2 KiB runs out, through
+// LDS, the byte transpose in registers (16 dwords of 4 k each -> 4 x 16 bytes, by 4 x 4 byte transposes). HBM-bound:
+// 13.4 us for a 37.7 MB weight, 5.6 TB/s read and written.
+constexpr int kTileChunks = 8;                 // 128 k
+constexpr int kTileCols = 128;                 // 8 groups of 16 n
+constexpr int kGroupPitch = 16 * 16 + 128;     // LDS bytes of 16 columns of one chunk: neighbours 32 banks apart
+constexpr int kChunkPitch = 8 * kGroupPitch + 16;   // neighbouring chunks 4 banks apart
+
+// The dword's four e5m2 codes without the infinite ones (0x7c, 0xfc), which become zero.
+__device__ __forceinline__ uint32_t drop_e5m2_inf(uint32_t w) {
+    const uint32_t other = (((w & 0x7f7f7f7fu) ^ 0x7c7c7c7cu) + 0x7f7f7f7fu) & 0x80808080u;   // set where not inf
+    return w & ((other >> 7) * 0xffu);
+}
+
+// The place of 16-byte unit k of a group's 128: the writes below take every fourth unit, the reads consecutive ones,
+// and both spread over all banks.
+__device__ __forceinline__ uint32_t swizzled_unit(uint32_t k) {
+    return (k & ~3u) | ((k ^ (k >> 4)) & 3u);
+}
+
+__global__ __launch_bounds__(kThreads) void transpose_prepacked_kernel(const uint8_t* b, uint8_t* out, uint32_t K,
+                                                                        uint32_t N, uint32_t n16, uint32_t copies,
+                                                                        bool e5m2, uint32_t k_tiles) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kTileChunks * kChunkPitch];
+    const uint32_t t = threadIdx.x;
+    const uint32_t chunk0 = blockIdx.x % k_tiles * kTileChunks;
+    const uint32_t n0 = blockIdx.x / k_tiles * kTileCols;
+    const uint32_t chunks = K / 16u;
+    const rsrc_t src = make_rsrc(b, chunks * N * 16u);
+    const rsrc_t dst = make_rsrc(out, copies * n16 * K * 16u);
+    u32x4 in[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t chunk = chunk0 + t / kTileCols + 2u * i;
+        const uint32_t n = n0 + t % kTileCols;
+        in[i] = buf_load16(src, chunk < chunks && n < N ? (chunk * N + n) * 16u : kOob);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t n = t % kTileCols;
+        *reinterpret_cast<u32x4*>(lds + (t / kTileCols + 2u * i) * kChunkPitch + n / 16u * kGroupPitch + n % 16u * 16u) =
+            in[i];
+    }
+    __syncthreads();
+    // Work-item t: columns 16 (t / 32) .. + 15, k values 4 (t % 32) .. + 3 of the tile.
+    const uint32_t group = t / 32u;
+    const uint32_t k4 = t % 32u;
+    uint32_t o[4][4];   // [k][4 columns]
+    const uint8_t* base = lds + k4 / 4u * kChunkPitch + group * kGroupPitch + k4 % 4u * 4u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        uint32_t d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = *reinterpret_cast<const uint32_t*>(base + (4 * r + i) * 16);
+        const uint32_t a0 = __builtin_amdgcn_perm(d[1], d[0], perm_sel(0, 4, 1, 5));
+        const uint32_t a1 = __builtin_amdgcn_perm(d[1], d[0], perm_sel(2, 6, 3, 7));
+        const uint32_t c0 = __builtin_amdgcn_perm(d[3], d[2], perm_sel(0, 4, 1, 5));
+        const uint32_t c1 = __builtin_amdgcn_perm(d[3], d[2], perm_sel(2, 6, 3, 7));
+        o[0][r] = __builtin_amdgcn_perm(c0, a0, perm_sel(0, 1, 4, 5));
+        o[1][r] = __builtin_amdgcn_perm(c0, a0, perm_sel(2, 3, 6, 7));
+        o[2][r] = __builtin_amdgcn_perm(c1, a1, perm_sel(0, 1, 4, 5));
+        o[3][r] = __builtin_amdgcn_perm(c1, a1, perm_sel(2, 3, 6, 7));
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        *reinterpret_cast<u32x4*>(lds + group * 2048u + swizzled_unit(4u * k4 + j) * 16u) =
+            u32x4{o[j][0], o[j][1], o[j][2], o[j][3]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t g = t / 128u + 2u * i;
+        const uint32_t k = t % 128u;
+        u32x4 v = *reinterpret_cast<const u32x4*>(lds + g * 2048u + swizzled_unit(k) * 16u);
+        const uint32_t ng = n0 / 16u + g;
+        const uint32_t kk = chunk0 * 16u + k;
+        for (uint32_t c = 0; c < copies; ++c) {
+            const uint32_t off = ng < n16 && kk < K ? ((c * n16 + ng) * K + kk) * 16u : kOob;
+            __builtin_amdgcn_raw_buffer_store_b128(v, dst, static_cast<int>(off), 0, 0);
+            if (e5m2 && c == 0) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) v[w] = drop_e5m2_inf(v[w]);
+            }
+        }
+    }
+}
+
+// ---- per-column scales -----------------------------------------------------------------------------------------
+
+// h (24 significant bits) = t[0] + t[1] + t[2], bf16 bits each, by truncation: exact, and t[0] never overflows. Of
+// inf and NaN the first term carries everything.
+__device__ __forceinline__ void split3(float h, uint32_t (&t)[3]) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, h);
+    const bool finite = (bits & 0x7f800000u) != 0x7f800000u;
+    // a NaN whose payload lies in the low half keeps being one
+    t[0] = (bits >> 16) | ((bits & 0x7fffffffu) > 0x7f800000u ? 0x40u : 0u);
+    const float r1 = h - __builtin_bit_cast(float, bits & 0xffff0000u);
+    const uint32_t bits1 = __builtin_bit_cast(uint32_t, r1);
+    const float r2 = r1 - __builtin_bit_cast(float, bits1 & 0xffff0000u);
+    t[1] = finite ? bits1 >> 16 : 0u;
+    t[2] = finite ? __builtin_bit_cast(uint32_t, r2) >> 16 : 0u;
+}
+
+// g [M, N] times scale [N] -> out [M, 3 Nc] bf16, Nc = 16 * ceil(N / 16): the three terms of column n at n, Nc + n
+// and 2 Nc + n, zero past N. One work-item per 8 columns: 16 bytes in, 3 x 16 out. HBM-bound.
+template <bool kBf16>
+__global__ __launch_bounds__(kThreads) void split_columns_kernel(const uint16_t* g, const float* scale, uint16_t* out,
+                                                                  uint32_t M, uint32_t N, uint32_t nc) {
+    const uint32_t pieces = nc / 8u;
+    const uint32_t piece = blockIdx.x * kThreads + threadIdx.x;
+    const uint32_t row = piece / pieces;
+    const uint32_t col = piece % pieces * 8u;
+    if (row >= M) return;
+    const bool in = col < N;
+    const rsrc_t src = make_rsrc(g, M * N * 2u);
+    const rsrc_t scale_rsrc = make_rsrc(scale, N * 4u);
+    const rsrc_t dst = make_rsrc(out, M * nc * 6u);
+    const u32x4 v = buf_load16(src, in ? (row * N + col) * 2u : kOob);
+    const f32x4 s0 = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, in ? col * 4u : kOob));
+    const f32x4 s1 = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, in ? col * 4u + 16u : kOob));
+    u32x4 t[3];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const uint32_t pair = v[w];
+        float lo, hi;
+        if constexpr (kBf16) {
+            lo = __builtin_bit_cast(float, pair << 16);
+            hi = __builtin_bit_cast(float, pair & 0xffff0000u);
+        } else {
+            const half2v h = __builtin_bit_cast(half2v, pair);
+            lo = static_cast<float>(h[0]);
+            hi = static_cast<float>(h[1]);
+        }
+        const float sl = w < 2 ? s0[2 * w] : s1[2 * w - 4];
+        const float sh = w < 2 ? s0[2 * w + 1] : s1[2 * w - 3];
+        uint32_t tl[3], th[3];
+        split3(lo * sl, tl);
+        split3(hi * sh, th);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) t[i][w] = tl[i] | (th[i] << 16);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 3; ++i) {
+        __builtin_amdgcn_raw_buffer_store_b128(t[i], dst, static_cast<int>((row * 3u * nc + i * nc + col) * 2u), 0, 0);
+    }
+}
+
+// ---- column sums -----------------------------------------------------------------------------------------------
+
+constexpr uint32_t kSumCols = 256;    // columns of a workgroup: 32 work-items x 8
+constexpr uint32_t kSumLanes = 8;     // rows summed side by side
+constexpr uint32_t kSumMinRows = 32;  // rows of a workgroup, at least
+
+template <bool kBf16>
+__device__ __forceinline__ uint16_t round16(float x) {
+    return static_cast<uint16_t>(pack_out<kBf16>(x, x) & 0xffffu);
+}
+
+// Rows [y R, (y + 1) R) of 256 columns -> partial [y][N] fp32, or, alone (one slab of rows), `out`. HBM-bound: each
+// work-item keeps four 16-byte loads in flight (4096 x 12288: 17.4 us, 5.8 TB/s, against 272 for torch's sum). All sums
+// in fp32, in a fixed order.
+template <bool kBf16>
+__global__ __launch_bounds__(kThreads) void column_sums_kernel(const uint16_t* g, float* partial, uint16_t* out,
+                                                                uint32_t M, uint32_t N, uint32_t rows) {
+    __shared__ float red[kSumLanes][kSumCols];
+    const rsrc_t src = make_rsrc(g, M * N * 2u);
+    const uint32_t lane = threadIdx.x / 32u;
+    const uint32_t col_in = threadIdx.x % 32u * 8u;
+    const uint32_t col = blockIdx.x * kSumCols + col_in;
+    const uint32_t end = min(M, (blockIdx.y + 1) * rows);
+    float sum[8] = {};
+    constexpr int kUnroll = 4;
+    for (uint32_t row = blockIdx.y * rows + lane; row < end; row += kUnroll * kSumLanes) {
+        u32x4 v[kUnroll];
+#pragma unroll
+        for (uint32_t i = 0; i < kUnroll; ++i) {
+            const uint32_t r = row + i * kSumLanes;
+            v[i] = buf_load16(src, r < end && col < N ? (r * N + col) * 2u : kOob);
+        }
+#pragma unroll
+        for (int i = 0; i < kUnroll; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint32_t pair = v[i][w];
+                if constexpr (kBf16) {
+                    sum[2 * w] += __builtin_bit_cast(float, pair << 16);
+                    sum[2 * w + 1] += __builtin_bit_cast(float, pair & 0xffff0000u);
+                } else {
+                    const half2v h = __builtin_bit_cast(half2v, pair);
+                    sum[2 * w] += static_cast<float>(h[0]);
+                    sum[2 * w + 1] += static_cast<float>(h[1]);
+                }
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) red[lane][col_in + i] = sum[i];
+    __syncthreads();
+    const uint32_t c = blockIdx.x * kSumCols + threadIdx.x;
+    if (c >= N) return;
+    float total = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kSumLanes; ++i) total += red[i][threadIdx.x];
+    if (gridDim.y == 1) {
+        out[c] = round16<kBf16>(total);
+    } else {
+        partial[blockIdx.y * N + c] = total;
+    }
+}
+
+template <bool kBf16>
+__global__ __launch_bounds__(kThreads) void column_sums_join_kernel(const float* partial, uint16_t* out, uint32_t N,
+                                                                     uint32_t slabs) {
+    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+    if (c >= N) return;
+    float total = 0.f;
+    for (uint32_t s = 0; s < slabs; ++s) total += partial[s * N + c];
+    out[c] = round16<kBf16>(total);
+}
+
+// Slabs of rows of the column sums: about four workgroups per CU, at least kSumMinRows rows each.
+int64_t sum_slabs(int64_t M, int64_t N) {
+    const int64_t col_tiles = (N + kSumCols - 1) / kSumCols;
+    return std::max<int64_t>(1, std::min<int64_t>((1024 + col_tiles - 1) / col_tiles, M / kSumMinRows));
+}
+
+// ---- workspace -------------------------------------------------------------------------------------------------
+
+constexpr int64_t align256(int64_t n) {
+    return (n + 255) / 256 * 256;
+}
+
+struct Layout {
+    int64_t depth;         // the matmul's contraction: N, or 3 * 16 * ceil(N / 16) with per-column scales
+    int64_t weight;        // bytes of the transposed weight, at 0
+    int64_t terms;         // of the split gradient, after it
+    int64_t sums;          // of the column sums' partials, after that
+    int64_t total() const { return weight + terms + sums; }
+};
+
+Layout layout(int64_t M, int64_t N, int64_t K, bool per_column) {
+    const int64_t n16 = (N + 15) / 16;
+    Layout l{};
+    l.depth = per_column ? 3 * 16 * n16 : N;
+    l.weight = align256((l.depth + 127) / 128 * 8 * K * 16);
+    l.terms = per_column ? align256(M * l.depth * 2) : 0;
+    l.sums = align256(sum_slabs(M, N) * N * 4);
+    return l;
+}
+
+bool aligned16(const void* p) {
+    return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+}
+
+}  // namespace
+}  // namespace feather
+
+extern "C" int64_t feather_linear_backward_depth(const int64_t N, const bool per_column) {
+    return feather::layout(1, N, 16, per_column).depth;
+}
+
+extern "C" int64_t feather_linear_backward_workspace_bytes(const int64_t M, const int64_t N, const int64_t K,
+                                                           const bool per_column) {
+    if (M < 1 || N < 8 || N % 8 != 0 || K < 16 || K % 16 != 0) return -1;
+    constexpr int64_t most = (int64_t{1} << 31) - 1;   // buffer offsets
+    const feather::Layout l = feather::layout(M, N, K, per_column);
+    if (M * N * 2 > most || M * K * 2 > most || l.weight > most || l.terms > most || l.sums > most) return -1;
+    return l.total();
+}
+
+extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_t* const b_prepacked,
+                                        const float* const scale, uint16_t* const grad_x, uint16_t* const grad_bias,
+                                        const int64_t M, const int64_t N, const int64_t K, const bool per_column,
+                                        const bool use_fp8_e5m2, const bool bf16, const int block_warps_m,
+                                        const int block_warps_n, const int unroll_k, const int repeat_m,
+                                        const int repeat_n, const bool prefetch, const int splits,
+                                        void* const split_workspace, const int64_t split_workspace_bytes,
+                                        void* const workspace, const int64_t workspace_bytes, hipStream_t stream) {
+    using namespace feather;
+    const int64_t need = feather_linear_backward_workspace_bytes(M, N, K, per_column);
+    if (need < 0 || !workspace || workspace_bytes < need || !aligned16(workspace)) return false;
+    if (!grad || !aligned16(grad) || (!grad_x && !grad_bias)) return false;
+    const Layout l = layout(M, N, K, per_column);
+    uint8_t* const weight = static_cast<uint8_t*>(workspace);
+    const uint32_t m = static_cast<uint32_t>(M), n = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
+    if (grad_x) {
+        if (!b_prepacked || !scale || !aligned16(b_prepacked) || !aligned16(grad_x)) return false;
+        if (per_column && !aligned16(scale)) return false;
+        const TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
+        const uint16_t* const operand = per_column ? reinterpret_cast<uint16_t*>(weight + l.weight) : grad;
+        if (!grad_matmul_ok(tile, M, K, l.depth, bf16 || per_column, splits, split_workspace, split_workspace_bytes)) {
+            return false;
+        }
+        const uint32_t n16 = (n + 15) / 16;
+        const uint32_t k_tiles = (k + 16 * kTileChunks - 1) / (16 * kTileChunks);
+        const uint32_t n_tiles = (n + kTileCols - 1) / kTileCols;
+        hipLaunchKernelGGL(transpose_prepacked_kernel, dim3(k_tiles * n_tiles), dim3(kThreads), 0, stream, b_prepacked,
+                           weight, k, n, n16, per_column ? 3u : 1u, use_fp8_e5m2,
+                           k_tiles);
+        if (per_column) {
+            uint16_t* const terms = reinterpret_cast<uint16_t*>(weight + l.weight);
+            const uint32_t blocks = static_cast<uint32_t>((M * 2 * n16 + kThreads - 1) / kThreads);
+            hipLaunchKernelGGL(bf16 ? split_columns_kernel<true> : split_columns_kernel<false>, dim3(blocks),
+                               dim3(kThreads), 0, stream, grad, scale, terms, m, n, 16 * n16);
+        }
+        if (!launch_grad_matmul(tile, operand, weight, per_column ? nullptr : scale, grad_x, M, K, l.depth,
+                                use_fp8_e5m2, bf16 || per_column, bf16, splits, split_workspace, stream)) {
+            return false;
+        }
+    }
+    if (grad_bias) {
+        float* const partial = reinterpret_cast<float*>(weight + l.weight + l.terms);
+        const int64_t slabs = sum_slabs(M, N);
+        const uint32_t rows = static_cast<uint32_t>((M + slabs - 1) / slabs);
+        const uint32_t used = (m + rows - 1) / rows;
+        hipLaunchKernelGGL(bf16 ? column_sums_kernel<true> : column_sums_kernel<false>,
+                           dim3((n + kSumCols - 1) / kSumCols, used), dim3(kThreads), 0, stream, grad, partial,
+                           grad_bias, m, n, rows);
+        if (used > 1) {
+            hipLaunchKernelGGL(bf16 ? column_sums_join_kernel<true> : column_sums_join_kernel<false>,
+                               dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, partial, grad_bias, n,
+                               used);
+        }
+    }
+    return true;
+}

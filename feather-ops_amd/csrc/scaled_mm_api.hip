@@ -74,6 +74,15 @@ bool is_tile(int wm, int wn, int u, int rm, int rn, bool prefetch) {
 #undef FEATHER_IS_TILE
 }
 
+// True for a tile of the gradient matmul's bf16 instantiations.
+bool is_grad_tile(const TileQuery& t) {
+#define FEATHER_IS_GRAD_TILE(twm, twn, tu, trm, trn, tpf)                                              \
+    || (((tpf) != 0) == t.prefetch && t.warps_m == (twm) && t.warps_n == (twn) && t.unroll_k == (tu) && \
+        t.repeat_m == (trm) && t.repeat_n == (trn))
+    return false FEATHER_GRAD_TILES(FEATHER_IS_GRAD_TILE);
+#undef FEATHER_IS_GRAD_TILE
+}
+
 // Workspace of a split launch: the counter area (one uint32 per tile and join slot, at most kSplitCtrBytes),
 // then the partial sums (splits fp32 tiles per output tile); none for splits = 1. -1 when the tile, the
 // split count or the grid is out of contract. A ring tile joins per wave (WM * WN slots) and splits its
@@ -193,6 +202,31 @@ Params make_params(const uint16_t* a, const uint8_t* b_prepacked, const float* s
 }
 
 }  // namespace
+
+bool grad_matmul_ok(const TileQuery& t, int64_t M, int64_t K, int64_t depth, bool operand_bf16, int splits,
+                    const void* split_workspace, int64_t split_workspace_bytes) {
+    if (depth < 16 || depth % 8 != 0 || depth * M * 2 > kMaxBufferBytes) return false;
+    const SplitLayout l =
+        split_layout(M, K, depth, t.warps_m, t.warps_n, t.unroll_k, t.repeat_m, t.repeat_n, t.prefetch, splits);
+    if (l.total_bytes < 0 || (operand_bf16 && !is_grad_tile(t))) return false;
+    return splits == 1 || (split_workspace && aligned(split_workspace, 256) && split_workspace_bytes >= l.total_bytes);
+}
+
+bool launch_grad_matmul(const TileQuery& t, const uint16_t* operand, const uint8_t* b, const float* scale,
+                        uint16_t* grad_x, int64_t M, int64_t K, int64_t depth, bool use_fp8_e5m2, bool operand_bf16,
+                        bool out_bf16, int splits, void* split_workspace, hipStream_t stream) {
+    Params p = make_params(operand, b, scale, nullptr, grad_x, M, K, depth, scale ? 1 : 0, 0);
+    p.stream_weight = 0;   // the transposed weight was written just before: it comes from the caches
+    if (splits > 1) {
+        p.splits = splits;
+        p.split_ctr = static_cast<uint32_t*>(split_workspace);
+        p.split_part = static_cast<uint8_t*>(split_workspace) + kSplitCtrBytes;
+    }
+    if (!operand_bf16) return use_fp8_e5m2 ? launch_combo_100(t, p, stream) : launch_combo_000(t, p, stream);
+    if (use_fp8_e5m2) return out_bf16 ? launch_combo_121(t, p, stream) : launch_combo_120(t, p, stream);
+    return out_bf16 ? launch_combo_021(t, p, stream) : launch_combo_020(t, p, stream);
+}
+
 }  // namespace feather
 
 extern "C" bool launch_scaled_mm(const uint16_t* const a, const uint8_t* const b_prepacked, const float* const scale,

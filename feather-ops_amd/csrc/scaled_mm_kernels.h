@@ -126,13 +126,29 @@ __device__ __forceinline__ void e4m3x4_to_f16(uint32_t p, uint32_t& lo, uint32_t
     hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p, 1.0f, true));
 }
 
-// 16 weight bytes (16 consecutive k of one column) -> the two 8-wide fp16 MFMA operands.
-template <bool kE5M2>
-__device__ __forceinline__ void decode_chunk(const u32x4 raw, half8& first, half8& second) {
+// Two of a dword's four fp8 codes (its low or high pair) -> two bf16, times the power of two `pow2` (exact: a code
+// has at most 4 significant bits, and every e5m2 or e4m3fn value times 2^-100 .. 2^100 is a bf16 normal; inf and
+// NaN stay).
+template <bool kE5M2, bool kHi>
+__device__ __forceinline__ uint32_t fp8x2_to_bf16(uint32_t p, float pow2) {
+    if constexpr (kE5M2) {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(p, pow2, kHi));
+    } else {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(p, pow2, kHi));
+    }
+}
+
+// 16 weight bytes (16 consecutive k of one column) -> the two 8-wide MFMA operands: fp16, or bf16 times `pow2`
+// (kBf16Mfma).
+template <bool kE5M2, bool kBf16Mfma = false>
+__device__ __forceinline__ void decode_chunk(const u32x4 raw, half8& first, half8& second, float pow2 = 1.0f) {
     uint32_t d[8];
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        if constexpr (kE5M2) {
+        if constexpr (kBf16Mfma) {
+            d[2 * w] = fp8x2_to_bf16<kE5M2, false>(raw[w], pow2);
+            d[2 * w + 1] = fp8x2_to_bf16<kE5M2, true>(raw[w], pow2);
+        } else if constexpr (kE5M2) {
             e5m2x4_to_f16(raw[w], d[2 * w], d[2 * w + 1]);
         } else {
             e4m3x4_to_f16(raw[w], d[2 * w], d[2 * w + 1]);
@@ -204,14 +220,39 @@ __device__ __forceinline__ u32x2 epilogue4(const f32x4 acc, f32x4 scale, bool ha
     return has_bias ? out4<kOutBf16, true>(acc, scale, bias_bits) : out4<kOutBf16, false>(acc, scale, bias_bits);
 }
 
+// kBf16Mfma: the operands' bits are bf16 (carried as half8).
+template <bool kBf16Mfma = false>
 __device__ __forceinline__ f32x4 mfma16(half8 w, half8 x, f32x4 acc) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0);
+    if constexpr (kBf16Mfma) {
+        using bf16x8 = __bf16 __attribute__((ext_vector_type(8)));
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x),
+                                                       acc, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0);
+    }
 }
 
 // The per-tensor weight scale, read once at kernel start so that its latency hides under the main loop
 // (1 when there is none or the scales are per column).
 __device__ __forceinline__ float load_scale(const Params& p) {
     return p.scale && !p.col_scale ? *p.scale : 1.0f;
+}
+
+// kBf16Mfma: the per-tensor scale as a power of two that the weight's decode applies (returned) and the rest
+// (`scale`, in [1, 2) up to its sign), which the epilogue applies: the accumulators then hold sums of the
+// dequantized weight's size, so they overflow only where the result itself does. Scales outside 2^-100 .. 2^100
+// (zero, inf and NaN among them) stay whole in the epilogue.
+template <bool kBf16Mfma>
+__device__ __forceinline__ float split_pow2(float& scale) {
+    if constexpr (kBf16Mfma) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, scale);
+        const uint32_t exponent = (bits >> 23) & 0xffu;
+        if (exponent >= 27u && exponent <= 227u) {
+            scale = __builtin_bit_cast(float, (bits & 0x807fffffu) | (127u << 23));
+            return __builtin_bit_cast(float, exponent << 23);
+        }
+    }
+    return 1.0f;
 }
 
 // Per-column scales of the 4 columns each lane stores in each of a wave's RN column tiles (16-byte loads:
@@ -565,8 +606,10 @@ constexpr int lds_epilogue_bytes() {
 // join code (its partial reads raise register pressure: measured 3% slower on a 128 x 256 tile).
 // kDeep: the deep-ring variant of a 64-row tile (DmaShape), chosen by the launcher for small grids.
 // kNtWeight: the weight's direct loads carry the non-temporal hint (launches that read the weight once).
+// kBf16Mfma: the activations are bf16 and go to bf16 MFMAs as they are (the gradient matmul); with kABf16 instead
+// they are widened to fp16 first.
 template <int WM, int WN, int U, int RM, int RN, bool kE5M2, bool kABf16, bool kOutBf16, bool kSplitK, bool kDeep,
-          bool kNtWeight = false>
+          bool kNtWeight = false, bool kBf16Mfma = false>
 __global__ __launch_bounds__(kWave * WM * WN)
 __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPerEu))) void ring_dma_kernel(
     const Params p) {
@@ -594,26 +637,29 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
 
     const rsrc_t a_rsrc = make_rsrc(p.a, static_cast<uint32_t>(p.M) * static_cast<uint32_t>(p.K) * 2u);
     const rsrc_t b_rsrc = make_rsrc(p.b, static_cast<uint32_t>(p.kb_total) * static_cast<uint32_t>(p.N) * 16u);
-    const int k_chunks = p.K / 16;
+    // K is a multiple of 8: the last chunk may hold one 8-wide activation unit (the weight's other half is zero).
+    const int k_units = p.K / 8;
+    const int k_chunks = (p.K + 15) / 16;
     // This workgroup's stages: global stages [stage0, stage0 + stages). Loads address global stages; the
     // ring slots and the wait schedule count local ones.
     const int stages_total = (p.K + 16 * U - 1) / (16 * U);
     const int stage0 = split * stages_total / splits;
     const int stages = (split + 1) * stages_total / splits - stage0;
-    const float scale = load_scale(p);
-    const int full_stages = k_chunks / U;  // stages with every chunk inside K
+    float scale = load_scale(p);
+    const float pow2 = split_pow2<kBf16Mfma>(scale);
+    const int full_stages = k_units / (2 * U);  // stages with every unit inside K
 
     // Direct loads: instruction i of this wave fills 1 KiB of LDS, lane l the l-th 16 bytes of it. The
     // per-lane offsets are for stage 0; a stage adds a scalar offset. Out-of-range rows and columns carry
     // kOob, which stays past the buffer's end whatever is added.
     uint32_t a_off[S::kAInstr];
-    int a_chunk[S::kAInstr];
+    int a_unit[S::kAInstr];
 #pragma unroll
     for (int i = 0; i < S::kAInstr; ++i) {
         const int unit = (wave + i * S::kWaves) * kWave + lane;
         const int row = unit / S::kUnitsPerRow;
         const int u = a_unit_phys<S::kUnitsPerRow>(row, unit % S::kUnitsPerRow);  // XOR is its own inverse
-        a_chunk[i] = u >> 1;
+        a_unit[i] = u;
         const int grow = m0 + row;
         a_off[i] = grow < p.M ? (static_cast<uint32_t>(grow) * static_cast<uint32_t>(p.K) +
                                  static_cast<uint32_t>(u * 8)) * 2u
@@ -653,7 +699,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
         } else {
 #pragma unroll
             for (int i = 0; i < S::kAInstr; ++i) {
-                const bool ok = stage * U + a_chunk[i] < k_chunks;
+                const bool ok = stage * 2 * U + a_unit[i] < k_units;
                 a_regs[i] = buf_load16(a_rsrc, ok ? a_off[i] : kOob, soff);
             }
         }
@@ -675,7 +721,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
         } else {
 #pragma unroll
             for (int i = 0; i < S::kAInstr; ++i) {
-                const bool ok = stage * U + a_chunk[i] < k_chunks;
+                const bool ok = stage * 2 * U + a_unit[i] < k_units;
                 dma16(a_rsrc, base + (wave + i * S::kWaves) * 1024, ok ? a_off[i] : kOob, soff);
             }
         }
@@ -759,7 +805,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
         auto multiply_stage = [&](const StageOperands& op) {
             half8 w[2][RN];
 #pragma unroll
-            for (int j = 0; j < RN; ++j) decode_chunk<kE5M2>(op.b[j], w[0][j], w[1][j]);
+            for (int j = 0; j < RN; ++j) decode_chunk<kE5M2, kBf16Mfma>(op.b[j], w[0][j], w[1][j], pow2);
             // Each activation fragment feeds its RN MFMAs back to back, the weight fragment changing each time;
             // odd fragments take the weights in reverse, so one weight operand carries across the boundary
             // (~1% faster than restarting at j = 0; holding a weight fragment for RM MFMAs instead, or
@@ -773,7 +819,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
 #pragma unroll
                     for (int jj = 0; jj < RN; ++jj) {
                         const int j = (i & 1) ? RN - 1 - jj : jj;
-                        acc[i][j] = mfma16(w[s2][j], x, acc[i][j]);
+                        acc[i][j] = mfma16<kBf16Mfma>(w[s2][j], x, acc[i][j]);
                     }
                 }
         };
@@ -800,7 +846,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
 #pragma unroll
                         for (int j = 0; j < RN; ++j) {
                             half8 w0, w1;
-                            decode_chunk<kE5M2>(braw[j], w0, w1);
+                            decode_chunk<kE5M2, kBf16Mfma>(braw[j], w0, w1, pow2);
                             w[j] = s2 == 0 ? w0 : w1;
                         }
 #pragma unroll
@@ -810,7 +856,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
                             const half8 x =
                                 __builtin_bit_cast(half8, (kABf16 && !kStageA) ? bf16x8_to_f16x8(raw) : raw);
 #pragma unroll
-                            for (int j = 0; j < RN; ++j) acc[i][j] = mfma16(w[j], x, acc[i][j]);
+                            for (int j = 0; j < RN; ++j) acc[i][j] = mfma16<kBf16Mfma>(w[j], x, acc[i][j]);
                         }
                     }
                 }
@@ -918,7 +964,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
 #pragma unroll
                     for (int j = 0; j < RN; ++j) {
                         half8 w0, w1;
-                        decode_chunk<kE5M2>(braw[j], w0, w1);
+                        decode_chunk<kE5M2, kBf16Mfma>(braw[j], w0, w1, pow2);
                         w[j] = s2 == 0 ? w0 : w1;
                     }
 #pragma unroll
@@ -927,7 +973,7 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
                             a_stage + a_lane[q][s2] + i * 16 * S::kUnitsPerRow * 16);
                         const half8 x = __builtin_bit_cast(half8, (kABf16 && !kStageA) ? bf16x8_to_f16x8(raw) : raw);
 #pragma unroll
-                        for (int j = 0; j < RN; ++j) acc[i][j] = mfma16(w[j], x, acc[i][j]);
+                        for (int j = 0; j < RN; ++j) acc[i][j] = mfma16<kBf16Mfma>(w[j], x, acc[i][j]);
                     }
                 }
             }
@@ -1043,8 +1089,9 @@ struct StreamShape {
 };
 
 // kNtWeight: the weight loads carry the non-temporal hint (launches that read the weight once).
+// kBf16Mfma: as for the ring kernel.
 template <int KS, int WN, int U, int RM, int RN, bool kE5M2, bool kABf16, bool kOutBf16, bool kSplitK,
-          bool kNtWeight = false>
+          bool kNtWeight = false, bool kBf16Mfma = false>
 __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p) {
     using S = StreamShape<KS, WN, U, RM, RN>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::kLdsBytes];
@@ -1055,7 +1102,8 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     const int ks = wave / WN;          // which K slice this wave reduces
     const int wave_n = wave % WN;
 
-    const float scale = load_scale(p);
+    float scale = load_scale(p);
+    const float pow2 = split_pow2<kBf16Mfma>(scale);
     const int tiles_n = (p.N + S::kBN - 1) / S::kBN;
     // A split launch runs `splits` workgroups per tile, split-major (as the ring kernel's split launch).
     const int n_tiles = ((p.M + S::kBM - 1) / S::kBM) * tiles_n;
@@ -1073,7 +1121,8 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
 
     const int g = lane >> 4;
     const int r16 = lane & 15;
-    const int k_chunks = p.K / 16;
+    const int k_units = p.K / 8;               // K is a multiple of 8 (see the ring kernel)
+    const int k_chunks = (p.K + 15) / 16;
     const int groups_total = (k_chunks + 3) / 4;   // 64-deep groups covering K
     // This workgroup's groups [group0, group_end): all of them, or its split's share. Chunks from chunk_end
     // on read as zeros (the end of K, or the next split's range).
@@ -1081,6 +1130,7 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     const int group0 = split * groups_total / splits;
     const int group_end = (split + 1) * groups_total / splits;
     const int chunk_end = kSplitK ? min(k_chunks, 4 * group_end) : k_chunks;
+    const int unit_end = kSplitK ? min(k_units, 8 * group_end) : k_units;
 
     // Activation fragments reach this wave's LDS buffer by direct loads of whole 128-byte row segments
     // (one instruction: 8 rows x 8 units of 16 bytes, unit = 8 consecutive k), so every cache line an
@@ -1089,12 +1139,12 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     // slot l % 8 of row 8h + l / 8; a_dma[i][h] is its row's offset plus the unit's, kOob past M.
     uint8_t* const a_lds = lds + wave * S::kAWaveBytes;
     uint32_t a_dma[RM][2];
-    int a_dma_chunk[2];
+    int a_dma_unit[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int row_in = 8 * h + (lane >> 3);
         const int unit = (lane & 7) ^ a_swizzle_key<8>(row_in);
-        a_dma_chunk[h] = unit >> 1;
+        a_dma_unit[h] = unit;
 #pragma unroll
         for (int i = 0; i < RM; ++i) {
             const int row = m0 + 16 * i + row_in;
@@ -1136,7 +1186,7 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
             for (int i = 0; i < RM; ++i)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const bool ok = 4 * group + a_dma_chunk[h] < chunk_end;
+                    const bool ok = 8 * group + a_dma_unit[h] < unit_end;
                     dma16(a_rsrc, dst + i * S::kAFragBytes + h * 1024, ok ? a_dma[i][h] : kOob, a_soff);
                 }
             const int chunk = 4 * group + g;
@@ -1174,11 +1224,11 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
 #pragma unroll
             for (int j = 0; j < RN; ++j) {
                 half8 w0, w1;
-                decode_chunk<kE5M2>(f.b[q][j], w0, w1);
+                decode_chunk<kE5M2, kBf16Mfma>(f.b[q][j], w0, w1, pow2);
 #pragma unroll
                 for (int i = 0; i < RM; ++i) {
-                    acc[i][j] = mfma16(w0, xa[i][0], acc[i][j]);
-                    acc[i][j] = mfma16(w1, xa[i][1], acc[i][j]);
+                    acc[i][j] = mfma16<kBf16Mfma>(w0, xa[i][0], acc[i][j]);
+                    acc[i][j] = mfma16<kBf16Mfma>(w1, xa[i][1], acc[i][j]);
                 }
             }
         }

@@ -1,7 +1,8 @@
 // Instantiates every tile of feather_tiles.h for ONE (weight format, activation dtype, output dtype)
 // combination and dispatches a tile query to it. The build compiles this file once per combination,
-// with FEATHER_B_E5M2, FEATHER_A_BF16 and FEATHER_OUT_BF16 set to 0 or 1, so the eight combinations
-// compile in parallel. The instantiation flow (X-macro tile list -> template per tile) follows the
+// with FEATHER_B_E5M2, FEATHER_A_BF16 and FEATHER_OUT_BF16 set to 0 or 1, so the combinations compile in
+// parallel. FEATHER_A_BF16 = 2 is the gradient matmul's: bf16 operands go to bf16 MFMAs unwidened, on the tiles
+// its picks can name (FEATHER_GRAD_TILES). The instantiation flow (X-macro tile list -> template per tile) follows the
 // reference's dispatch_scaled_mm (csrc/hip_kernel.cu:668-684).
 #include "scaled_mm_launch.h"
 
@@ -10,14 +11,15 @@
 #include "scaled_mm_wide.h"
 
 #if !defined(FEATHER_B_E5M2) || !defined(FEATHER_A_BF16) || !defined(FEATHER_OUT_BF16)
-#error "compile with -DFEATHER_B_E5M2=<0|1> -DFEATHER_A_BF16=<0|1> -DFEATHER_OUT_BF16=<0|1>"
+#error "compile with -DFEATHER_B_E5M2=<0|1> -DFEATHER_A_BF16=<0|1|2> -DFEATHER_OUT_BF16=<0|1>"
 #endif
 
 namespace feather {
 namespace {
 
 constexpr bool kE5M2 = FEATHER_B_E5M2 != 0;
-constexpr bool kABf16 = FEATHER_A_BF16 != 0;
+constexpr bool kABf16 = FEATHER_A_BF16 == 1;
+constexpr bool kBf16Mfma = FEATHER_A_BF16 == 2;
 constexpr bool kOutBf16 = FEATHER_OUT_BF16 != 0;
 constexpr int kCus = 256;                // MI355X compute units
 
@@ -29,24 +31,25 @@ void launch_ring(const Params& q, dim3 grid, hipStream_t stream) {
     using S = DmaShape<WM, WN, U, RM, RN>;
     if constexpr (S::kBM <= 64) {
         if (q.stream_weight && q.M <= S::kBM) {
-            hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep, true>),
+            hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep, true,
+                                                kBf16Mfma>),
                                grid, dim3(S::kThreads), 0, stream, q);
             return;
         }
     }
-    hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep>), grid,
-                       dim3(S::kThreads), 0, stream, q);
+    hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep, false, kBf16Mfma>),
+                       grid, dim3(S::kThreads), 0, stream, q);
 }
 
 template <int KS, int WN, int U, int RM, int RN, bool kSplitK>
 void launch_stream(const Params& p, dim3 grid, hipStream_t stream) {
     using S = StreamShape<KS, WN, U, RM, RN>;
     if (p.stream_weight && p.M <= S::kBM) {
-        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, true>), grid,
-                           dim3(S::kThreads), 0, stream, p);
+        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, true, kBf16Mfma>),
+                           grid, dim3(S::kThreads), 0, stream, p);
     } else {
-        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK>), grid,
-                           dim3(S::kThreads), 0, stream, p);
+        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, false, kBf16Mfma>),
+                           grid, dim3(S::kThreads), 0, stream, p);
     }
 }
 
@@ -66,14 +69,14 @@ bool try_tile(const TileQuery& t, const Params& p, hipStream_t stream) {
         const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(S::kThreads), 0, stream, p); };
         if (p.splits > 1) {
             if (ragged) {
-                go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, true, true>);
+                go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, true, true, kBf16Mfma>);
             } else {
-                go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, true, false>);
+                go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, true, false, kBf16Mfma>);
             }
         } else if (ragged) {
-            go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, false, true>);
+            go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, false, true, kBf16Mfma>);
         } else {
-            go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, false, false>);
+            go(wide_kernel<RN, kE5M2, kABf16, kOutBf16, false, false, kBf16Mfma>);
         }
     } else if constexpr (PF != 0) {
         using S = DmaShape<WM, WN, U, RM, RN>;
@@ -136,7 +139,11 @@ bool try_tile(const TileQuery& t, const Params& p, hipStream_t stream) {
 bool FEATHER_COMBO_FN(FEATHER_B_E5M2, FEATHER_A_BF16, FEATHER_OUT_BF16)(const TileQuery& t, const Params& p,
                                                                           hipStream_t stream) {
 #define FEATHER_TRY_TILE(wm, wn, u, rm, rn, pf) || try_tile<wm, wn, u, rm, rn, pf>(t, p, stream)
+#if FEATHER_A_BF16 == 2
+    return false FEATHER_GRAD_TILES(FEATHER_TRY_TILE);
+#else
     return false FEATHER_SCALED_MM_TILES(FEATHER_TRY_TILE);
+#endif
 #undef FEATHER_TRY_TILE
 }
 

@@ -98,8 +98,10 @@ __device__ __forceinline__ uint32_t decode_word_(uint32_t w) {
     }
 }
 
-template <bool kE5M2>
-__device__ __forceinline__ uint32_t decode_word(uint32_t w, bool hi) {
+// kBf16Mfma: two bf16 values times `pow2` instead.
+template <bool kE5M2, bool kBf16Mfma>
+__device__ __forceinline__ uint32_t decode_word(uint32_t w, bool hi, float pow2) {
+    if constexpr (kBf16Mfma) return hi ? fp8x2_to_bf16<kE5M2, true>(w, pow2) : fp8x2_to_bf16<kE5M2, false>(w, pow2);
     return hi ? decode_word_<kE5M2, true>(w) : decode_word_<kE5M2, false>(w);
 }
 
@@ -165,7 +167,8 @@ __device__ __forceinline__ void store_wave_tiles_swap(const Params& p, const f32
 // kRagged: M % 256, N % kBN or K % 64 is not zero. Then every direct load masks its lanes (rows past M, columns
 // past N and chunks past K read zeros). Otherwise every load is whole and in range: the per-lane offsets are fixed
 // and the tile and stage go in the scalar offset.
-template <int RN_, bool kE5M2, bool kABf16, bool kOutBf16, bool kSplitK, bool kRagged>
+// kBf16Mfma: as for the ring kernel.
+template <int RN_, bool kE5M2, bool kABf16, bool kOutBf16, bool kSplitK, bool kRagged, bool kBf16Mfma = false>
 __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void wide_kernel(
     const Params p) {
     using S = WideShape<RN_>;
@@ -193,26 +196,28 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
     const int stages_total = (p.K + 63) / 64;
     const int stage0 = split * stages_total / splits;
     const int stages = (split + 1) * stages_total / splits - stage0;
-    const int k_chunks = p.K / 16;
+    const int k_units = p.K / 8;   // K is a multiple of 8 (see the ring kernel)
+    const int k_chunks = (p.K + 15) / 16;
 
     const rsrc_t a_rsrc = make_rsrc(p.a, static_cast<uint32_t>(p.M) * static_cast<uint32_t>(p.K) * 2u);
     const rsrc_t b_rsrc = make_rsrc(p.b, static_cast<uint32_t>(p.kb_total) * static_cast<uint32_t>(p.N) * 16u);
     const rsrc_t null_rsrc = make_rsrc(p.a, 0u);
-    const float scale = load_scale(p);
+    float scale = load_scale(p);
+    const float pow2 = split_pow2<kBf16Mfma>(scale);
 
     // Direct loads (the ring kernel's layout): load d < 8 of this wave fills 1 KiB of a slot's activations (8 rows
     // of 8 units: row (wave + 4d) * 8 + lane / 8 of the tile, physical unit lane % 8), load 8 + i fills the slot's
     // weight pieces e * 64 + lane, e = wave + 4i, of its [4 chunks][kBN columns] (kBN a multiple of 64, so one
-    // load covers 64 columns of one chunk). Per-lane offsets within the tile and stage; the unit's k chunk (the
+    // load covers 64 columns of one chunk). Per-lane offsets within the tile and stage; the unit's place in the stage (the
     // same for every d: the swizzle key depends on the row mod 16 only).
     uint32_t a_lane_off[S::kAInstr];
-    int a_chunk = 0;
+    int a_unit = 0;
 #pragma unroll
     for (int d = 0; d < S::kAInstr; ++d) {
         const int unit = (wave + d * S::kWaves) * kWave + lane;
         const int row = unit / S::kUnitsPerRow;
         const int u = a_unit_phys<S::kUnitsPerRow>(row, unit % S::kUnitsPerRow);
-        a_chunk = u >> 1;
+        a_unit = u;
         a_lane_off[d] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.K) + static_cast<uint32_t>(u * 8)) * 2u;
     }
     const int a_row_in = lane / S::kUnitsPerRow + wave * S::kUnitsPerRow;   // + 32 d: the row of load d
@@ -244,7 +249,7 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
         if (d < S::kAInstr) {
             uint8_t* dst = lds + slot + (wave + d * S::kWaves) * 1024;
             if constexpr (kRagged) {
-                const bool ok = m0 + a_row_in + 32 * d < p.M && a_chunk < k_chunks - 4 * stage;
+                const bool ok = m0 + a_row_in + 32 * d < p.M && a_unit < k_units - 8 * stage;
                 dma16(live ? a_rsrc : null_rsrc, dst, ok ? a_tile_off + a_lane_off[d] : kOob,
                       live ? static_cast<uint32_t>(stage) * 128u : 0u);
             } else {
@@ -303,7 +308,7 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
 #pragma unroll
     for (int j = 0; j < RN; ++j)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) w0[j][d] = decode_word<kE5M2>(braw[j][d / 2], d & 1);
+        for (int d = 0; d < 4; ++d) w0[j][d] = decode_word<kE5M2, kBf16Mfma>(braw[j][d / 2], d & 1, pow2);
 
     uint32_t cur = 0;                           // slot of stage t
     uint32_t nxt = S::kStageBytes;              // slot of stage t + 1
@@ -315,12 +320,12 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
             const int i = m / RN;
             const int jj = m % RN;
             const int j = (i & 1) ? RN - 1 - jj : jj;
-            acc[i][j] = mfma16(__builtin_bit_cast(half8, u32x4{w0[j][0], w0[j][1], w0[j][2], w0[j][3]}), as_f16(x0[i]),
-                               acc[i][j]);
+            acc[i][j] = mfma16<kBf16Mfma>(__builtin_bit_cast(half8, u32x4{w0[j][0], w0[j][1], w0[j][2], w0[j][3]}),
+                                          as_f16(x0[i]), acc[i][j]);
             if (jj == 0) x1[i] = read16(cur + a_rd1 + i * 2048);
             if (m >= S::kDecode1) {
                 const int q = m - S::kDecode1;  // 4 RN dwords of second-half weights, one per MFMA
-                w1[q / 4][q % 4] = decode_word<kE5M2>(braw[q / 4][2 + (q % 4) / 2], q & 1);
+                w1[q / 4][q % 4] = decode_word<kE5M2, kBf16Mfma>(braw[q / 4][2 + (q % 4) / 2], q & 1, pow2);
             }
             if (m >= S::kLateAt && (m - S::kLateAt) % S::kLateStep == 0 &&
                 (m - S::kLateAt) / S::kLateStep < S::kLoadsPerStage - S::kLoadsEarly) {
@@ -334,8 +339,8 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
             const int i = m / RN;
             const int jj = m % RN;
             const int j = (i & 1) ? RN - 1 - jj : jj;
-            acc[i][j] = mfma16(__builtin_bit_cast(half8, u32x4{w1[j][0], w1[j][1], w1[j][2], w1[j][3]}), as_f16(x1[i]),
-                               acc[i][j]);
+            acc[i][j] = mfma16<kBf16Mfma>(__builtin_bit_cast(half8, u32x4{w1[j][0], w1[j][1], w1[j][2], w1[j][3]}),
+                                          as_f16(x1[i]), acc[i][j]);
             if (m == 7) {
                 // This wave's reads of slot t % 3 are complete and its loads of stage t + 1 have landed (those of
                 // stage t + 2 may still be in flight); the barrier makes every wave's share of stage t + 1 visible,
@@ -352,8 +357,9 @@ __global__ __launch_bounds__(WideShape<RN_>::kThreads) __attribute__((amdgpu_wav
             }
             if (m >= S::kDecode0) {
                 const int q = 2 * (m - S::kDecode0);  // 4 RN dwords of stage t + 1's first-half weights, two per MFMA
-                w0[q / 4][q % 4] = decode_word<kE5M2>(braw[q / 4][(q % 4) / 2], q & 1);
-                w0[(q + 1) / 4][(q + 1) % 4] = decode_word<kE5M2>(braw[(q + 1) / 4][((q + 1) % 4) / 2], (q + 1) & 1);
+                w0[q / 4][q % 4] = decode_word<kE5M2, kBf16Mfma>(braw[q / 4][(q % 4) / 2], q & 1, pow2);
+                w0[(q + 1) / 4][(q + 1) % 4] =
+                    decode_word<kE5M2, kBf16Mfma>(braw[(q + 1) / 4][((q + 1) % 4) / 2], (q + 1) & 1, pow2);
             }
             __builtin_amdgcn_sched_barrier(0);
         }

@@ -39,6 +39,10 @@ def c_library() -> ctypes.CDLL:
         lib = ctypes.CDLL(str(LIBRARY))
         lib.feather_set_weight_streaming.restype = ctypes.c_int
         lib.feather_set_weight_streaming.argtypes = [ctypes.c_int]
+        lib.feather_linear_backward_workspace_bytes.restype = ctypes.c_int64
+        lib.feather_linear_backward_workspace_bytes.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool]
+        lib.feather_linear_backward_depth.restype = ctypes.c_int64
+        lib.feather_linear_backward_depth.argtypes = [ctypes.c_int64, ctypes.c_bool]
         _c_library = lib
     return _c_library
 

@@ -116,16 +116,21 @@ def _linear_setup_context(ctx, inputs, output) -> None:
 
 
 def _linear_backward(ctx, grad: torch.Tensor):
-    """Gradients for the activations and the bias (the fp8 weight is frozen): dX = dY @ (Wq * scale)^T in
-    fp32 on the dequantized weight, dbias = the column sums of dY."""
+    """Gradients for the activations and the bias (the fp8 weight is frozen): dX = dY @ (Wq * scale)^T as fp32
+    arithmetic gives it on the dequantized weight, dbias = the column sums of dY."""
+    from .linear_backward import composite, linear_backward
+
     weight_fp8, weight_scale = ctx.saved_tensors
     k = ctx.x_shape[-1]
-    chunks, n, _ = weight_fp8.shape
-    w = weight_fp8.permute(0, 2, 1).reshape(chunks * 16, n)[:k].float() * weight_scale.float()  # [K, N]
-    g = grad.reshape(-1, n).float()
-    grad_x = (g @ w.t()).to(ctx.x_dtype).reshape(ctx.x_shape)
-    grad_bias = None if ctx.bias_dtype is None else g.sum(0).to(ctx.bias_dtype)
-    return grad_x, None, None, grad_bias
+    need_x, need_bias = ctx.needs_input_grad[0], ctx.bias_dtype is not None and ctx.needs_input_grad[3]
+    # A gradient that is itself differentiated (create_graph) or batched by a transform (vmap, grad of grad) takes
+    # torch's operations, which have rules for both.
+    if (torch.is_grad_enabled() and grad.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(grad):
+        grad_x, grad_bias = composite(grad, weight_fp8, weight_scale, k)
+    else:
+        grad_x, grad_bias = linear_backward(grad, weight_fp8, weight_scale, k, need_x, need_bias)
+    return (grad_x.to(ctx.x_dtype).reshape(ctx.x_shape) if need_x else None, None, None,
+            grad_bias.to(ctx.bias_dtype) if need_bias else None)
 
 
 _scaled_mm_linear.register_autograd(_linear_backward, setup_context=_linear_setup_context)

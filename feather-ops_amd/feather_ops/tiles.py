@@ -57,6 +57,24 @@ SCALED_MM_TILES = [
     (2, 2, 4, 4, 2, 0),  # 64 x 64
 ]
 
+# The tiles the gradient matmul runs with bf16 operands (`csrc/linear_backward.hip`): those the heuristic returns for
+# fp16 activations, which is what it is asked for (the 256 x 256 ring tile's model time is never under 128 x 256's).
+GRAD_TILES = [
+    (1, 4, 4, 8, 4, 1),
+    (2, 2, 4, 8, 8, 1),
+    (2, 2, 4, 8, 6, 1),
+    (2, 2, 4, 4, 4, 1),
+    (1, 4, 4, 4, 2, 1),
+    (2, 2, 4, 2, 2, 1),
+    (2, 2, 4, 2, 2, 0),
+    (4, 1, 4, 1, 4, 0),
+    (4, 1, 8, 1, 4, 0),
+    (4, 1, 4, 1, 2, 0),
+    (8, 1, 4, 1, 2, 0),
+    (4, 1, 4, 1, 1, 0),
+    (8, 1, 4, 1, 1, 0),
+]
+
 
 def gemm_block_sizes(tile: tuple[int, ...]) -> tuple[int, int, int]:
     """`(block_m, block_n, chunk_k)` of a `SCALED_MM_TILES` entry."""

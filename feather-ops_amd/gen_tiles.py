@@ -1,4 +1,4 @@
-"""Render `feather_ops/tiles.py:SCALED_MM_TILES` into `csrc/feather_tiles.h`, or `--check` it is current.
+"""Render the tile tables of `feather_ops/tiles.py` into `csrc/feather_tiles.h`, or `--check` it is current.
 
 Mirrors the reference's `tools/gen_tiles.py:36-69` flow (render / --check) for the gfx950 table. The tiles
 module is loaded by path so this runs without torch or a built extension.
@@ -22,16 +22,17 @@ def load_tiles():
 
 
 def render() -> str:
-    tiles = load_tiles().SCALED_MM_TILES
+    tables = load_tiles()
     lines = [
         "// Generated by feather-ops_amd/gen_tiles.py from feather_ops/tiles.py. Do not edit.",
         "#pragma once",
         "",
         "// X(warps_m, warps_n, unroll_k, repeat_m, repeat_n, prefetch)",
-        "#define FEATHER_SCALED_MM_TILES(X) \\",
     ]
-    lines += [f"    X({', '.join(str(v) for v in tile)}) \\" for tile in tiles]
-    lines.append("")
+    for macro, tiles in (("SCALED_MM_TILES", tables.SCALED_MM_TILES), ("GRAD_TILES", tables.GRAD_TILES)):
+        lines.append(f"#define FEATHER_{macro}(X) \\")
+        lines += [f"    X({', '.join(str(v) for v in tile)}) \\" for tile in tiles]
+        lines.append("")
     return "\n".join(lines) + "\n"
 
 

@@ -1,0 +1,54 @@
+"""The backward's host side on the CPU: every tile its picks can name is instantiated for bf16 operands, and operands the
+kernels do not take go to torch's operations with the same result."""
+
+import random
+
+import pytest
+import torch
+
+from feather_ops import linear_backward as lb
+from feather_ops import prepack_transpose
+from feather_ops.tiles import GRAD_TILES, SCALED_MM_TILES, split_workspace_bytes
+
+
+def test_grad_tiles_cover_the_picks():
+    rng = random.Random(0)
+    assert set(GRAD_TILES) <= set(SCALED_MM_TILES)
+    seen = set()
+    for _ in range(6000):
+        m = int(2 ** rng.uniform(0, 14))
+        n = 8 * int(2 ** rng.uniform(0, 11.5))
+        k = 16 * int(2 ** rng.uniform(0, 10.5))
+        if rng.random() < 0.3:    # whole tiles of the wide kernel
+            m, n, k = (-(-s // 256) * 256 for s in (m, n, k))
+        for column in (False, True):
+            plan = lb.backward_plan(m, n, k, column)
+            if plan is None:
+                continue
+            tile, splits, split_bytes, nbytes = plan
+            assert tile in GRAD_TILES, (m, n, k, tile)
+            depth = 48 * -(-n // 16) if column else n
+            assert splits == 1 or split_bytes == split_workspace_bytes(m, k, depth, tile, splits)
+            assert nbytes >= -(-depth // 128) * 128 * k + (2 * m * depth if column else 0)
+            seen.add(tile)
+    assert seen == set(GRAD_TILES)
+
+
+def test_plan_refuses_buffers_past_2_gib():
+    assert lb.backward_plan(65536, 8192, 4096, True) is None      # the split gradient: 3.2 GB
+    assert lb.backward_plan(65536, 8192, 4096, False) is not None
+
+
+@pytest.mark.parametrize("column", [False, True])
+def test_operands_off_the_gpu_take_torch(column):
+    torch.manual_seed(0)
+    wq = torch.randn(24, 48).to(torch.float8_e5m2)
+    scale = torch.rand(24) + 0.5 if column else torch.tensor(0.5)
+    grad = torch.randn(2, 5, 24).to(torch.bfloat16)
+    x, bias = lb.linear_backward(grad, prepack_transpose(wq), scale, 48, True, True)
+    w = wq.float() * (scale[:, None] if column else scale)
+    want = grad.reshape(10, 24).float() @ w
+    assert x.shape == (10, 48) and (x.float() - want).abs().max() <= 2.0**-8 * want.abs().max()
+    assert torch.equal(bias, grad.reshape(10, 24).float().sum(0).to(torch.bfloat16))
+    none_x, none_b = lb.linear_backward(grad, prepack_transpose(wq), scale, 48, False, False)
+    assert none_x.numel() == none_b.numel() == 0

@@ -243,6 +243,55 @@ void prepack_b(const Tensor& b, Tensor& out) {
     STD_TORCH_CHECK(err == hipSuccess, "prepack_b kernel launch failed: ", hipGetErrorString(err));
 }
 
+// What prepack_rows and quantize_rows share: w [N, K] -> out [K_pad/16, N, 16] fp8, both contiguous on one device.
+void check_rows(const Tensor& w, const Tensor& out) {
+    STD_TORCH_CHECK(w.is_cuda() && out.is_cuda() && w.get_device_index() == out.get_device_index(),
+                    "w and out must be CUDA tensors on one device");
+    STD_TORCH_CHECK(out.scalar_type() == ST::Float8_e5m2 || out.scalar_type() == ST::Float8_e4m3fn,
+                    "out must be float8_e5m2 or float8_e4m3fn");
+    STD_TORCH_CHECK(w.dim() == 2 && out.dim() == 3 && w.is_contiguous() && out.is_contiguous(),
+                    "w must be a contiguous [N, K] and out a contiguous [K_pad/16, N, 16] tensor");
+    STD_TORCH_CHECK(out.size(0) == (w.size(1) + 127) / 128 * 8 && out.size(1) == w.size(0) && out.size(2) == 16,
+                    "out must be [ceil(K/128)*8, N, 16]");
+}
+
+// feather_ops::prepack_rows: an fp8 weight [N, K] laid out (feather_prepack_rows).
+void prepack_rows(const Tensor& w, Tensor& out) {
+    check_rows(w, out);
+    STD_TORCH_CHECK(w.scalar_type() == out.scalar_type(), "out must have w's dtype");
+    const auto device_index = w.get_device_index();
+    torch::stable::accelerator::DeviceGuard guard(device_index);
+    check_launch(feather_prepack_rows(static_cast<const uint8_t*>(w.const_data_ptr()),
+                                      static_cast<uint8_t*>(out.mutable_data_ptr()), w.size(0), w.size(1),
+                                      current_stream(device_index)),
+                 "prepack_rows");
+}
+
+// feather_ops::quantize_rows: a bf16, fp16 or fp32 weight [N, K] quantized and laid out (feather_quantize_rows); scale of
+// N elements (per row) or one, amax int32 scratch.
+void quantize_rows(const Tensor& w, Tensor& out, Tensor& scale, Tensor& amax) {
+    check_rows(w, out);
+    const auto device_index = w.get_device_index();
+    const int64_t N = w.size(0);
+    const auto type = w.scalar_type();
+    STD_TORCH_CHECK(type == ST::BFloat16 || type == ST::Half || type == ST::Float,
+                    "w must be bfloat16, float16 or float32");
+    STD_TORCH_CHECK(scale.is_cuda() && scale.get_device_index() == device_index && scale.scalar_type() == ST::Float &&
+                        scale.is_contiguous() && (scale.dim() == 0 || (scale.dim() == 1 && scale.numel() == N)),
+                    "scale must be float32 on w's device, one value (0-D) or N (1-D)");
+    STD_TORCH_CHECK(amax.is_cuda() && amax.get_device_index() == device_index && amax.scalar_type() == ST::Int &&
+                        amax.is_contiguous() && amax.numel() >= N && amax.numel() >= 1024,
+                    "amax must be int32 on w's device, max(N, 1024) elements");
+    torch::stable::accelerator::DeviceGuard guard(device_index);
+    check_launch(feather_quantize_rows(w.const_data_ptr(), type == ST::BFloat16 ? 0 : type == ST::Half ? 1 : 2,
+                                       static_cast<uint8_t*>(out.mutable_data_ptr()),
+                                       static_cast<float*>(scale.mutable_data_ptr()),
+                                       static_cast<uint32_t*>(amax.mutable_data_ptr()), N, w.size(1),
+                                       out.scalar_type() == ST::Float8_e5m2, scale.dim() == 1,
+                                       current_stream(device_index)),
+                 "quantize_rows");
+}
+
 // feather_ops::linear_backward: feather_linear_backward on tensors (grad [M, N], b_prepacked [K_pad/16, N, 16], scale of
 // one or N elements; grad_x [M, K] and grad_bias [N] in grad's dtype, each optional). split_workspace: as
 // scaled_mm_splitk's, ignored for splits = 1. workspace: uint8, any content.
@@ -315,6 +364,8 @@ STABLE_TORCH_LIBRARY(feather_ops, m) {
     m.def("bf16_to_fp16(Tensor x, Tensor(a!) out) -> ()");
     m.def("widen_bf16(Tensor x, Tensor(a!) out) -> ()");
     m.def("prepack_b(Tensor b, Tensor(a!) out) -> ()");
+    m.def("prepack_rows(Tensor w, Tensor(a!) out) -> ()");
+    m.def("quantize_rows(Tensor w, Tensor(a!) out, Tensor(b!) scale, Tensor(c!) amax) -> ()");
     m.def(
         "linear_backward(Tensor grad, Tensor b_prepacked, Tensor scale, Tensor(a!)? grad_x, Tensor(b!)? grad_bias, "
         "Tensor(c!) split_workspace, Tensor(d!) workspace, int K, int splits, int block_warps_m, int block_warps_n, "
@@ -327,6 +378,8 @@ STABLE_TORCH_LIBRARY_IMPL(feather_ops, CUDA, m) {
     m.impl("bf16_to_fp16", TORCH_BOX(&bf16_to_fp16));
     m.impl("widen_bf16", TORCH_BOX(&widen_bf16));
     m.impl("prepack_b", TORCH_BOX(&prepack_b));
+    m.impl("prepack_rows", TORCH_BOX(&prepack_rows));
+    m.impl("quantize_rows", TORCH_BOX(&quantize_rows));
     m.impl("linear_backward", TORCH_BOX(&linear_backward));
 }
 

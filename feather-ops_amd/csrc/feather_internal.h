@@ -38,6 +38,21 @@ int64_t feather_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K,
 /* The inputs (contraction length) of feather_linear_backward's matmul: what its tile and splits are chosen for. */
 int64_t feather_linear_backward_depth(int64_t N, bool per_column);
 
+/*
+ * w [N, K] row-major -> out [K_pad/16][N][16], zero-padded to K_pad = ceil(K / 128) * 128: the layout of
+ * feather_prepack_b for a weight stored as a Linear stores it. Requires K % 16 == 0, 16-byte aligned pointers and
+ * both buffers under 2 GiB; returns false (nothing enqueued) otherwise.
+ */
+bool feather_prepack_rows(const uint8_t* w, uint8_t* out, int64_t N, int64_t K, hipStream_t stream);
+
+/*
+ * The same for a weight to quantize (source 0: bf16, 1: fp16, 2: fp32): per row (scale holds N values) or per tensor
+ * (one), scale = amax / the format's largest value, 1 where amax is zero or NaN, codes = w / scale rounded to nearest
+ * even. amax: scratch of max(N, 1024) words, any content. Same contract; w's buffer under 2 GiB too.
+ */
+bool feather_quantize_rows(const void* w, int source, uint8_t* out, float* scale, uint32_t* amax, int64_t N, int64_t K,
+                           bool use_fp8_e5m2, bool per_row, hipStream_t stream);
+
 }  // extern "C"
 
 #endif  // FEATHER_INTERNAL_H

@@ -63,9 +63,15 @@ class ScaledMMLinear:
     """
 
     def quantize_weight_(self, fp8_dtype: torch.dtype = torch.float8_e5m2, per_channel: bool = False) -> None:
-        from .scaled_mm import prepack_transpose
+        from .scaled_mm import prepack_transpose, quantize_and_pack
 
-        w = self.weight.detach().float()
+        w = self.weight.detach()
+        packed = quantize_and_pack(w, fp8_dtype, per_channel)
+        if packed is not None:
+            self.register_buffer("weight_fp8", packed[0], persistent=False)
+            self.register_buffer("weight_scale", packed[1], persistent=False)
+            return
+        w = w.float()
         amax = w.abs().amax(dim=1) if per_channel else w.abs().max().reshape(1)
         scale = torch.where(amax > 0, amax / _FP8_MAX[fp8_dtype], torch.ones_like(amax))
         wq = (w / (scale[:, None] if per_channel else scale)).to(fp8_dtype)

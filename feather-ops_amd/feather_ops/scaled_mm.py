@@ -757,11 +757,14 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
 
     `K` is zero-padded to a multiple of 128, so a ragged K never needs a staging branch; element
     `[k // 16, n, k % 16]` of the result is `b[k, n]`. A contiguous e5m2 / e4m3fn weight on the GPU with
-    N a multiple of 8 is permuted by one HIP kernel (`csrc/prepack.hip`, HBM-bound); anything else
-    (a CPU weight, another dtype or width) by torch copy kernels on `b`'s device. Run once per weight.
+    N a multiple of 8 is permuted by one HIP kernel (`csrc/prepack.hip`, HBM-bound), and so is the transposed
+    view of a contiguous `[N, K]` one with K a multiple of 16; anything else (a CPU weight, another dtype or
+    width) by torch copy kernels on `b`'s device. Run once per weight.
     """
     k, n = b.shape
     k_pad = -(-k // 128) * 128
+    if b.dtype in _FP8_DTYPES and _packs_rows(b.t()):
+        return prepack_transpose(b.t())
     if (b.is_cuda and b.dtype in (torch.float8_e5m2, torch.float8_e4m3fn) and b.is_contiguous()
             and n % 8 == 0 and n > 0 and k > 0 and b.data_ptr() % 8 == 0):
         out = torch.empty((k_pad // 16, n, 16), device=b.device, dtype=b.dtype)
@@ -774,16 +777,50 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
     return b.view(k_pad // 16, 16, n).permute(0, 2, 1).contiguous()
 
 
+def _packs_rows(w: torch.Tensor) -> bool:
+    """Whether the row-packing kernels take `w` [N, K]: an fp8 (to lay out), bf16, fp16 or fp32 (to quantize) weight on
+    the GPU, its rows whole 16-byte units and its buffers under 2 GiB; a plain tensor, outside tracing and
+    transforms, whose copies autograd does not follow."""
+    return (w.is_cuda and w.dim() == 2 and w.dtype in _PACKED_DTYPES and w.is_contiguous() and w.numel() > 0
+            and w.shape[1] % 16 == 0 and type(w) in (torch.Tensor, torch.nn.Parameter)
+            and not torch.compiler.is_compiling() and not torch._C._functorch.is_functorch_wrapped_tensor(w)
+            and w.data_ptr() % 16 == 0 and w.shape[0] * (-(-w.shape[1] // 128) * 128) * w.element_size() < 1 << 31
+            and not (w.requires_grad and torch.is_grad_enabled()))
+
+
+def quantize_and_pack(w: torch.Tensor, fp8_dtype: torch.dtype,
+                      per_channel: bool) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """(`[K_pad/16, N, 16]` codes, scale) of a bf16, fp16 or fp32 weight `[N, K]` on the GPU, in two passes over it; None
+    where the kernels do not take it. The scale is N values (per channel) or one (0-D)."""
+    if w.dtype in _FP8_DTYPES or fp8_dtype not in _FP8_DTYPES or not _packs_rows(w):
+        return None
+    n, k = w.shape
+    out = torch.empty((-(-k // 128) * 8, n, 16), device=w.device, dtype=fp8_dtype)
+    scale = torch.empty(n if per_channel else (), device=w.device, dtype=torch.float32)
+    amax = torch.empty(max(n, 1024), device=w.device, dtype=torch.int32)
+    torch.ops.feather_ops.quantize_rows.default(w, out, scale, amax)
+    return out, scale
+
+
+_FP8_DTYPES = (torch.float8_e5m2, torch.float8_e4m3fn)
+_PACKED_DTYPES = _FP8_DTYPES + (torch.bfloat16, torch.float16, torch.float32)
+
+
 def prepack_transpose(w: torch.Tensor) -> torch.Tensor:
     """`[N, K]` fp8 weight (an `nn.Linear` weight, out x in) -> `[K_pad/16, N, 16]`: the same layout as
     `prepack_b_for_scaled_mm(w.t())` without materializing the transpose (the external consumer's
     `comfy_feather/quant.py::prepack_transpose`, named at the reference's `scaled_mm.py:141-142`).
 
     For a row of `w` the 16 k values of a chunk are already 16 contiguous bytes, so the prepack is a
-    transpose of `[N, K_pad/16]` 16-byte units.
+    transpose of `[N, K_pad/16]` 16-byte units: one HIP kernel (`csrc/prepack.hip`) where it takes the weight
+    (`_packs_rows`), torch copies otherwise.
     """
     n, k = w.shape
     k_pad = -(-k // 128) * 128
+    if w.dtype in _FP8_DTYPES and _packs_rows(w):
+        out = torch.empty((k_pad // 16, n, 16), device=w.device, dtype=w.dtype)
+        torch.ops.feather_ops.prepack_rows.default(w, out)
+        return out
     if k_pad != k:
         padded = torch.zeros((n, k_pad), device=w.device, dtype=w.dtype)
         padded[:, :k] = w

@@ -613,6 +613,77 @@ def _auto_choice(M: int, N: int, K: int,
     return tile, select_scaled_mm_splits(M, N, K, tile, a_dtype), False
 
 
+# A few rows past a multiple of the tile's rows (a prompt's 16 text rows after the image tokens, one class token) cost a
+# whole row of tiles, and with it often another round on every CU: 4112 x 12288 x 4096 runs 1056 tiles of 128 x 128, 4.1
+# per CU, in 348 us, 4096 rows of it one round of 256 x 256 tiles in 248. From _TAIL_MIN_GAIN of predicted gain on, the
+# last M % 256 or M % 128 rows (at most _TAIL_MAX_ROWS) get a launch of their own on their own pick, which reads the
+# weight once more. Predictions are microseconds fitted on 150 shapes (M 256-9232, N 1024-16384, K 1536-14208; each
+# tile within 5% in standard deviation): per 64-deep stage and round of resident blocks, one round with `last` blocks a
+# CU instead of the `resident` ones, per block of a CU, and once. Rows of _LARGE_TIME: resident, stage times with 1 ..
+# resident blocks, block, once.
+# Of 41 shapes with 1-64 such rows where fp16 (or widened) launches pass the line, the split measured 0.99-1.34x, 1.13x
+# in geometric mean (4112 x 12288 x 4096 1.33, 4097 x 2560 x 5120 1.10); below it, at most 1.10x and down to 0.84.
+_LARGE_TIME = {
+    _TILE_WIDE: ((1.10,), 16.4, -8.75),
+    _TILE_WIDE_192: ((0.942,), 9.66, -3.5),
+    _TILE_RING_128x256_W64: ((0.903, 1.168), 4.41, -0.3),
+    _TILE_RING_128x128: ((0.498, 0.682, 1.129), 0.836, 2.46),
+    _TILE_RING_64x128: ((0.217, 0.515, 0.659), 0.614, 1.93),
+}
+_TAIL_MAX_ROWS = 64
+_TAIL_MIN_GAIN = 1.10
+
+
+def _large_time(M: int, N: int, K: int, tile: tuple[int, ...], splits: int) -> float | None:
+    """Predicted microseconds of an unsplit launch with fp16 activations on a tile of _LARGE_TIME, else None."""
+    if splits != 1 or tile not in _LARGE_TIME:
+        return None
+    stage, block, once = _LARGE_TIME[tile]
+    per_cu = -(-_blocks(M, N, tile) // _CUS)
+    rounds, last = divmod(per_cu, len(stage))
+    return -(-K // 64) * (rounds * stage[-1] + (stage[last - 1] if last else 0.0)) + block * per_cu + once
+
+
+def _tail_time(rows: int, N: int, K: int) -> float:
+    """Predicted microseconds of the last rows' own launch: its weight read at 5 TB/s, once more or less in part from 17 and
+    from 33 rows on."""
+    return max(6.0, (3.0 + N * K / 5e6) * (1.0 if rows <= 16 else 1.35 if rows <= 32 else 1.8))
+
+
+@functools.lru_cache(maxsize=4096)
+def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tuple[int, tuple[int, ...], int], ...], bool]:
+    """The launches the auto path runs a shape as, ((rows, tile, splits), ...) from the first row on, and whether bf16
+    activations are widened first: `_auto_choice`'s single one, or two where the last few rows are better off alone."""
+    tile, splits, widen = _auto_choice(M, N, K, a_dtype)
+    whole = ((M, tile, splits),), widen
+    if M <= 256 or M % 128 == 0 or M % 128 > _TAIL_MAX_ROWS:
+        return whole
+    widen_us = max(_WIDEN_MIN_S, 4.0 * M * K / _WIDEN_BYTES_PER_S) * 1e6 if a_dtype == torch.bfloat16 else 0.0
+    if a_dtype == torch.bfloat16 and not widen:
+        # in place: the fp16 form's time and its lead (`widen_first`)
+        fp16_tile = _TILE_RING_128x256_W64 if tile == _TILE_RING_128x256 else tile
+        lead = (_WIDEN_LEAD_W64 if fp16_tile == _TILE_RING_128x256_W64
+                else max(0.0, _WIDEN_LEAD_SMALL * (1.0 - _WIDEN_LEAD_SMALL_K0 / K)))
+        now = _large_time(M, N, K, fp16_tile, splits)
+        now = None if now is None else now * (1.0 + lead)
+    else:
+        now = _large_time(M, N, K, tile, splits)
+        now = None if now is None else now + widen_us
+    best = None
+    for rows in {M - M % 256, M - M % 128}:
+        if now is None or M - rows > _TAIL_MAX_ROWS:
+            continue
+        main = _auto_choice(rows, N, K, torch.float16)
+        time = _large_time(rows, N, K, *main[:2])
+        if time is None:
+            continue
+        time += _tail_time(M - rows, N, K) + widen_us
+        if now >= _TAIL_MIN_GAIN * time and (best is None or time < best[0]):
+            tail = _auto_choice(M - rows, N, K, torch.float16)
+            best = time, ((rows, *main[:2]), (M - rows, *tail[:2]))
+    return whole if best is None else (best[1], a_dtype == torch.bfloat16)
+
+
 # Split-K workspaces, one per (device, stream): the counter area at their start must be zero before a
 # launch, and every completed launch leaves it zero whatever its shape, so a workspace is zeroed once, when
 # it is created, and then reused by the launches of its stream, which are ordered. Other streams get their
@@ -673,6 +744,11 @@ def set_weight_streaming(mode: str | None = None) -> str:
     return _STREAMING_MODES[previous]
 
 
+def _whole_rows(a: torch.Tensor) -> bool:
+    """Whether activations are laid out as the op takes them."""
+    return a.is_cuda and a.dim() == 2 and a.is_contiguous() and a.numel() < (1 << 30)
+
+
 def _launch(
     a: torch.Tensor,
     b_prepacked: torch.Tensor,
@@ -683,12 +759,10 @@ def _launch(
     splits: int = 1,
     widen: bool = False,
 ) -> None:
-    if widen and a.is_cuda and a.dim() == 2 and a.is_contiguous() and a.numel() < (1 << 30):
-        # an fp16 copy of the bf16 activations, rounded as the kernels round them; activations the op would
-        # refuse are passed on as they are, so that it reports them as it does without the widening
-        wide = torch.empty(a.shape, dtype=torch.float16, device=a.device)
-        torch.ops.feather_ops.widen_bf16.default(a, wide)
-        a = wide
+    if widen and _whole_rows(a):
+        # activations the op would refuse are passed on as they are, so that it reports them as it does without
+        # the widening
+        a = _widened(a)
     if splits == 1:
         torch.ops.feather_ops.scaled_mm.default(a, b_prepacked, scale, bias, out, *tile)
         return
@@ -703,6 +777,31 @@ def _launch(
     torch.ops.feather_ops.scaled_mm_splitk.default(a, b_prepacked, scale, bias, out, ws, splits, *tile)
 
 
+def _widened(a: torch.Tensor) -> torch.Tensor:
+    """An fp16 copy of bf16 activations, rounded as the kernels round them."""
+    wide = torch.empty(a.shape, dtype=torch.float16, device=a.device)
+    torch.ops.feather_ops.widen_bf16.default(a, wide)
+    return wide
+
+
+def _launch_auto(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bias: torch.Tensor | None,
+                 out: torch.Tensor) -> None:
+    """The heuristic's launch or launches."""
+    parts, widen = _auto_parts(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype)
+    if len(parts) == 1 or not _whole_rows(a) or not out.is_contiguous():
+        # activations the op would refuse go to it as they are, in one launch, so that it reports them
+        _, tile, splits = parts[0] if len(parts) == 1 else (0, *_auto_choice(a.shape[0], b_prepacked.shape[1],
+                                                                             a.shape[1], a.dtype)[:2])
+        _launch(a, b_prepacked, scale, bias, out, tile, splits, widen)
+        return
+    if widen:
+        a = _widened(a)
+    row = 0
+    for rows, tile, splits in parts:
+        _launch(a[row:row + rows], b_prepacked, scale, bias, out[row:row + rows], tile, splits)
+        row += rows
+
+
 @custom_op("feather_ops::scaled_mm_auto", mutates_args=("out",))
 def _scaled_mm_auto(
     a: torch.Tensor,
@@ -713,7 +812,7 @@ def _scaled_mm_auto(
 ) -> None:
     """The auto-picked launch inside one custom op: a compiled graph holds a single node for it, whichever
     tile, split count or widening the shape leads to."""
-    _launch(a, b_prepacked, scale, bias, out, *_auto_choice(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype))
+    _launch_auto(a, b_prepacked, scale, bias, out)
 
 
 def scaled_mm_hip(
@@ -742,7 +841,7 @@ def scaled_mm_hip(
         if torch.compiler.is_compiling():
             _scaled_mm_auto(a, b_prepacked, scale, bias, out)
         else:
-            _launch(a, b_prepacked, scale, bias, out, *_auto_choice(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype))
+            _launch_auto(a, b_prepacked, scale, bias, out)
     else:
         if tile is None:
             tile = select_scaled_mm_config(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype,

@@ -1,0 +1,102 @@
+"""The auto path's second launch for a few last rows: which shapes take it (CPU), and its outputs (GPU)."""
+
+import random
+
+import pytest
+import torch
+
+from feather_ops.scaled_mm import _TAIL_MAX_ROWS, _auto_choice, _auto_parts
+
+FP16, BF16 = torch.float16, torch.bfloat16
+
+# (m, n, k): one row, 16 and 64 of them past a whole round of wide tiles, of 256 x 192 ones, of 128 x 128 and 64 x 128
+# ring tiles; a tail split along K; N off the tiles
+SPLIT = [(4097, 5120, 2560), (4112, 4096, 4096), (4160, 4096, 4096), (4112, 3072, 3072), (1281, 5960, 5248),
+         (1040, 4096, 12288), (2208, 3712, 2368)]
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("m,n,k", SPLIT)
+def test_shapes_that_split(m, n, k, dtype):
+    parts, widen = _auto_parts(m, n, k, dtype)
+    assert len(parts) == 2 and widen == (dtype == BF16)
+    assert parts[0] == (m - m % 128 if m % 256 > 64 else m - m % 256, *_auto_choice(parts[0][0], n, k, FP16)[:2])
+
+
+def test_parts_cover_the_rows_once():
+    rng = random.Random(0)
+    split = 0
+    for _ in range(20000):
+        m, n, k = int(2 ** rng.uniform(0, 14)), 8 * int(2 ** rng.uniform(0, 11)), 16 * int(2 ** rng.uniform(0, 10))
+        for dtype in (FP16, BF16):
+            parts, widen = _auto_parts.__wrapped__(m, n, k, dtype)
+            assert sum(rows for rows, _, _ in parts) == m
+            if len(parts) == 1:
+                assert (*parts[0][1:], widen) == _auto_choice(m, n, k, dtype)
+                continue
+            split += 1
+            (head, tile, splits), (tail, *tail_pick) = parts
+            assert head % 128 == 0 and splits == 1 and 0 < tail <= _TAIL_MAX_ROWS and m >= 320 - 64
+            assert (tile, splits) == _auto_choice(head, n, k, FP16)[:2]
+            assert tuple(tail_pick) == _auto_choice(tail, n, k, FP16)[:2]
+    assert split > 50
+    for m in (1, 77, 256, 512, 4096, 4224, 4096 + 100):
+        assert len(_auto_parts(m, 4096, 4096, FP16)[0]) == 1
+
+
+def _inputs(m, n, k, dtype, column):
+    import feather_ops
+
+    g = torch.Generator("cuda").manual_seed(m)
+    a = torch.randn((m, k), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 20).to(torch.float8_e4m3fn)
+    scale = (torch.rand(n, generator=g, device="cuda") + 0.5) * 1e-3 if column else torch.tensor(1e-3, device="cuda")
+    return a, feather_ops.prepack_transpose(w), scale, torch.randn(n, generator=g, device="cuda").to(dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("m,n,k", SPLIT)
+def test_outputs(m, n, k, dtype):
+    import feather_ops
+    from gpu_helpers import check_against_oracle
+
+    for column in (False, True):
+        a, b, scale, bias = _inputs(m, n, k, dtype, column)
+        out = feather_ops.scaled_mm_hip(a, b, scale, bias, dtype)
+        rows = sorted({0, 1, 255, 256, m // 2, *range(m - m % 128 - 2, m)})
+        check_against_oracle(out, a, b, scale, bias, rows=rows)
+
+
+@pytest.mark.gpu
+def test_graph_replays():
+    import feather_ops
+
+    m, n, k = SPLIT[5]      # the tail splits K: its workspace is part of the graph
+    a, b, scale, bias = _inputs(m, n, k, BF16, True)
+    inputs = [torch.randn_like(a) for _ in range(3)]
+    want = [feather_ops.scaled_mm_hip(x, b, scale, bias, BF16) for x in inputs]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = feather_ops.scaled_mm_hip(a, b, scale, bias, BF16)
+    for x, y in zip(inputs + inputs[:1], want + want[:1]):
+        a.copy_(x)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), y.view(torch.int16))
+        feather_ops.scaled_mm_hip(x, b, scale, bias, BF16)
+
+
+@pytest.mark.gpu
+def test_refused_operands_are_refused_as_before():
+    import feather_ops
+
+    a, b, scale, bias = _inputs(4112, 4096, 4096, FP16, False)
+    with pytest.raises(RuntimeError, match="stride"):
+        feather_ops.scaled_mm_hip(torch.cat([a, a], dim=1)[:, :4096], b, scale, bias, FP16)
+    with pytest.raises(RuntimeError, match="aligned"):
+        feather_ops.scaled_mm_hip(torch.empty(a.numel() + 1, device="cuda", dtype=FP16)[1:].view_as(a), b, scale, bias, FP16)
+    with pytest.raises(RuntimeError, match="bias"):
+        feather_ops.scaled_mm_hip(a, b, scale, bias.to(BF16), FP16)

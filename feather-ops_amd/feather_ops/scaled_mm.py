@@ -684,6 +684,16 @@ def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tup
     return whole if best is None else (best[1], a_dtype == torch.bfloat16)
 
 
+@functools.lru_cache(maxsize=4096)
+def _packed_tile(M: int, N: int, K: int, a_dtype: torch.dtype) -> int | None:
+    """The tile of a shape the auto path runs as one plain launch (unsplit, activations as given), its six numbers packed
+    into one for `feather_ops::scaled_mm_new`; None for the others."""
+    parts, widen = _auto_parts(M, N, K, a_dtype)
+    if widen or len(parts) > 1 or parts[0][2] > 1:
+        return None
+    return sum(field << 8 * i for i, field in enumerate(parts[0][1]))
+
+
 # Split-K workspaces, one per (device, stream): the counter area at their start must be zero before a
 # launch, and every completed launch leaves it zero whatever its shape, so a workspace is zeroed once, when
 # it is created, and then reused by the launches of its stream, which are ordered. Other streams get their
@@ -802,6 +812,10 @@ def _launch_auto(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor
         row += rows
 
 
+_lib.load()
+_scaled_mm_new = torch.ops.feather_ops.scaled_mm_new.default
+
+
 @custom_op("feather_ops::scaled_mm_auto", mutates_args=("out",))
 def _scaled_mm_auto(
     a: torch.Tensor,
@@ -833,11 +847,21 @@ def scaled_mm_hip(
     The heuristic's launch goes through the opaque custom op `feather_ops::scaled_mm_auto` while
     `torch.compile` traces (as in the reference, `scaled_mm.py:104-134`), and straight to the launcher in
     eager mode: the same launch without the custom op's Python dispatch, about 7 us of host time per call,
-    which is more than a decode-sized kernel takes.
+    which is more than a decode-sized kernel takes. Where that is one plain launch, one op allocates the output
+    and launches it.
     """
     _lib.require_native()
+    auto = tile is None and splits is None
+    if auto and (out_dtype is torch.bfloat16 or out_dtype is torch.float16) and not torch.compiler.is_compiling():
+        shape = a.shape
+        packed = _packed_tile(shape[0], b_prepacked.shape[1], shape[1], a.dtype)
+        # operands that autograd follows take the ops that write into an output: it marks what an op returns
+        if packed is not None and not (a.requires_grad or b_prepacked.requires_grad
+                                       or (scale is not None and scale.requires_grad)
+                                       or (bias is not None and bias.requires_grad)):
+            return _scaled_mm_new(a, b_prepacked, scale, bias, out_dtype is torch.bfloat16, packed)
     out = torch.empty((a.shape[0], b_prepacked.shape[1]), device=a.device, dtype=out_dtype)
-    if tile is None and splits is None:
+    if auto:
         if torch.compiler.is_compiling():
             _scaled_mm_auto(a, b_prepacked, scale, bias, out)
         else:
@@ -862,8 +886,8 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
     """
     k, n = b.shape
     k_pad = -(-k // 128) * 128
-    if b.dtype in _FP8_DTYPES and _packs_rows(b.t()):
-        return prepack_transpose(b.t())
+    if b.dtype in _FP8_DTYPES and b.stride(0) == 1 and _packs_rows(b.t()):
+        return _pack_rows(b.t())
     if (b.is_cuda and b.dtype in (torch.float8_e5m2, torch.float8_e4m3fn) and b.is_contiguous()
             and n % 8 == 0 and n > 0 and k > 0 and b.data_ptr() % 8 == 0):
         out = torch.empty((k_pad // 16, n, 16), device=b.device, dtype=b.dtype)
@@ -905,6 +929,13 @@ _FP8_DTYPES = (torch.float8_e5m2, torch.float8_e4m3fn)
 _PACKED_DTYPES = _FP8_DTYPES + (torch.bfloat16, torch.float16, torch.float32)
 
 
+def _pack_rows(w: torch.Tensor) -> torch.Tensor:
+    n, k = w.shape
+    out = torch.empty((-(-k // 128) * 8, n, 16), device=w.device, dtype=w.dtype)
+    torch.ops.feather_ops.prepack_rows.default(w, out)
+    return out
+
+
 def prepack_transpose(w: torch.Tensor) -> torch.Tensor:
     """`[N, K]` fp8 weight (an `nn.Linear` weight, out x in) -> `[K_pad/16, N, 16]`: the same layout as
     `prepack_b_for_scaled_mm(w.t())` without materializing the transpose (the external consumer's
@@ -917,9 +948,7 @@ def prepack_transpose(w: torch.Tensor) -> torch.Tensor:
     n, k = w.shape
     k_pad = -(-k // 128) * 128
     if w.dtype in _FP8_DTYPES and _packs_rows(w):
-        out = torch.empty((k_pad // 16, n, 16), device=w.device, dtype=w.dtype)
-        torch.ops.feather_ops.prepack_rows.default(w, out)
-        return out
+        return _pack_rows(w)
     if k_pad != k:
         padded = torch.zeros((n, k_pad), device=w.device, dtype=w.dtype)
         padded[:, :k] = w

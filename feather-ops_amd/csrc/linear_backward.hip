@@ -179,6 +179,18 @@ __global__ __launch_bounds__(kThreads) void split_columns_kernel(const uint16_t*
     }
 }
 
+// g [M, N] with N % 16 = 8 -> out [M, N + 8], zero in the new columns: the streaming kernel's rows are whole chunks.
+__global__ __launch_bounds__(kThreads) void pad_columns_kernel(const uint16_t* g, uint16_t* out, uint32_t M, uint32_t N) {
+    const uint32_t pieces = N / 8u + 1u;
+    const uint32_t piece = blockIdx.x * kThreads + threadIdx.x;
+    const uint32_t row = piece / pieces;
+    const uint32_t col = piece % pieces * 8u;
+    if (row >= M) return;
+    const u32x4 v = buf_load16(make_rsrc(g, M * N * 2u), col < N ? (row * N + col) * 2u : kOob);
+    __builtin_amdgcn_raw_buffer_store_b128(v, make_rsrc(out, M * (N + 8u) * 2u),
+                                           static_cast<int>((row * (N + 8u) + col) * 2u), 0, 0);
+}
+
 // ---- column sums -----------------------------------------------------------------------------------------------
 
 constexpr uint32_t kSumCols = 256;    // columns of a workgroup: 32 work-items x 8
@@ -266,7 +278,7 @@ constexpr int64_t align256(int64_t n) {
 struct Layout {
     int64_t depth;         // the matmul's contraction: N, or 3 * 16 * ceil(N / 16) with per-column scales
     int64_t weight;        // bytes of the transposed weight, at 0
-    int64_t terms;         // of the split gradient, after it
+    int64_t terms;         // of the split gradient, or of a padded one (N % 16 = 8), after it
     int64_t sums;          // of the column sums' partials, after that
     int64_t total() const { return weight + terms + sums; }
 };
@@ -276,7 +288,7 @@ Layout layout(int64_t M, int64_t N, int64_t K, bool per_column) {
     Layout l{};
     l.depth = per_column ? 3 * 16 * n16 : N;
     l.weight = align256((l.depth + 127) / 128 * 8 * K * 16);
-    l.terms = per_column ? align256(M * l.depth * 2) : 0;
+    l.terms = per_column ? align256(M * l.depth * 2) : N % 16 ? align256(M * 16 * n16 * 2) : 0;
     l.sums = align256(sum_slabs(M, N) * N * 4);
     return l;
 }
@@ -320,8 +332,11 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
         if (!b_prepacked || !scale || !aligned16(b_prepacked) || !aligned16(grad_x)) return false;
         if (per_column && !aligned16(scale)) return false;
         const TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
-        const uint16_t* const operand = per_column ? reinterpret_cast<uint16_t*>(weight + l.weight) : grad;
-        if (!grad_matmul_ok(tile, M, K, l.depth, bf16 || per_column, splits, split_workspace, split_workspace_bytes)) {
+        const bool pad = !prefetch && !per_column && N % 16 != 0;
+        const int64_t depth = pad ? N + 8 : l.depth;
+        uint16_t* const made = reinterpret_cast<uint16_t*>(weight + l.weight);
+        const uint16_t* const operand = per_column || pad ? made : grad;
+        if (!grad_matmul_ok(tile, M, K, depth, bf16 || per_column, splits, split_workspace, split_workspace_bytes)) {
             return false;
         }
         const uint32_t n16 = (n + 15) / 16;
@@ -331,12 +346,14 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
                            weight, k, n, n16, per_column ? 3u : 1u, use_fp8_e5m2,
                            k_tiles);
         if (per_column) {
-            uint16_t* const terms = reinterpret_cast<uint16_t*>(weight + l.weight);
             const uint32_t blocks = static_cast<uint32_t>((M * 2 * n16 + kThreads - 1) / kThreads);
             hipLaunchKernelGGL(bf16 ? split_columns_kernel<true> : split_columns_kernel<false>, dim3(blocks),
-                               dim3(kThreads), 0, stream, grad, scale, terms, m, n, 16 * n16);
+                               dim3(kThreads), 0, stream, grad, scale, made, m, n, 16 * n16);
+        } else if (pad) {
+            const uint32_t blocks = static_cast<uint32_t>((M * (N / 8 + 1) + kThreads - 1) / kThreads);
+            hipLaunchKernelGGL(pad_columns_kernel, dim3(blocks), dim3(kThreads), 0, stream, grad, made, m, n);
         }
-        if (!launch_grad_matmul(tile, operand, weight, per_column ? nullptr : scale, grad_x, M, K, l.depth,
+        if (!launch_grad_matmul(tile, operand, weight, per_column ? nullptr : scale, grad_x, M, K, depth,
                                 use_fp8_e5m2, bf16 || per_column, bf16, splits, split_workspace, stream)) {
             return false;
         }

@@ -637,7 +637,8 @@ __attribute__((amdgpu_waves_per_eu(DmaShape<WM, WN, U, RM, RN, kDeep>::kWavesPer
 
     const rsrc_t a_rsrc = make_rsrc(p.a, static_cast<uint32_t>(p.M) * static_cast<uint32_t>(p.K) * 2u);
     const rsrc_t b_rsrc = make_rsrc(p.b, static_cast<uint32_t>(p.kb_total) * static_cast<uint32_t>(p.N) * 16u);
-    // K is a multiple of 8: the last chunk may hold one 8-wide activation unit (the weight's other half is zero).
+    // K is a multiple of 8 (the streaming kernel's of 16): the last chunk may hold one 8-wide activation unit (the
+    // weight's other half is zero).
     const int k_units = p.K / 8;
     const int k_chunks = (p.K + 15) / 16;
     // This workgroup's stages: global stages [stage0, stage0 + stages). Loads address global stages; the
@@ -1121,8 +1122,7 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
 
     const int g = lane >> 4;
     const int r16 = lane & 15;
-    const int k_units = p.K / 8;               // K is a multiple of 8 (see the ring kernel)
-    const int k_chunks = (p.K + 15) / 16;
+    const int k_chunks = p.K / 16;
     const int groups_total = (k_chunks + 3) / 4;   // 64-deep groups covering K
     // This workgroup's groups [group0, group_end): all of them, or its split's share. Chunks from chunk_end
     // on read as zeros (the end of K, or the next split's range).
@@ -1130,7 +1130,6 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     const int group0 = split * groups_total / splits;
     const int group_end = (split + 1) * groups_total / splits;
     const int chunk_end = kSplitK ? min(k_chunks, 4 * group_end) : k_chunks;
-    const int unit_end = kSplitK ? min(k_units, 8 * group_end) : k_units;
 
     // Activation fragments reach this wave's LDS buffer by direct loads of whole 128-byte row segments
     // (one instruction: 8 rows x 8 units of 16 bytes, unit = 8 consecutive k), so every cache line an
@@ -1139,12 +1138,12 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     // slot l % 8 of row 8h + l / 8; a_dma[i][h] is its row's offset plus the unit's, kOob past M.
     uint8_t* const a_lds = lds + wave * S::kAWaveBytes;
     uint32_t a_dma[RM][2];
-    int a_dma_unit[2];
+    int a_dma_chunk[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int row_in = 8 * h + (lane >> 3);
         const int unit = (lane & 7) ^ a_swizzle_key<8>(row_in);
-        a_dma_unit[h] = unit;
+        a_dma_chunk[h] = unit >> 1;
 #pragma unroll
         for (int i = 0; i < RM; ++i) {
             const int row = m0 + 16 * i + row_in;
@@ -1186,7 +1185,7 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
             for (int i = 0; i < RM; ++i)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const bool ok = 8 * group + a_dma_unit[h] < unit_end;
+                    const bool ok = 4 * group + a_dma_chunk[h] < chunk_end;
                     dma16(a_rsrc, dst + i * S::kAFragBytes + h * 1024, ok ? a_dma[i][h] : kOob, a_soff);
                 }
             const int chunk = 4 * group + g;

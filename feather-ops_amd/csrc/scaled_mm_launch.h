@@ -36,7 +36,7 @@ bool launch_combo_120(const TileQuery&, const Params&, hipStream_t);
 bool launch_combo_121(const TileQuery&, const Params&, hipStream_t);
 
 // grad_x [M, K] = operand [M, depth] @ b [depth/16, K, 16] * scale (one value; none: 1), the gradient matmul of
-// linear_backward.hip: depth a multiple of 8, the operand bf16 (operand_bf16) or fp16, the output bf16 or fp16 (fp16
+// linear_backward.hip: depth a multiple of 8 (streaming tiles: 16), the operand bf16 (operand_bf16) or fp16, the output bf16 or fp16 (fp16
 // operands: fp16). `grad_matmul_ok` says on the host whether the tile, the splits and their workspace fit.
 bool grad_matmul_ok(const TileQuery& tile, int64_t M, int64_t K, int64_t depth, bool operand_bf16, int splits,
                     const void* split_workspace, int64_t split_workspace_bytes);

@@ -886,13 +886,13 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
     """
     k, n = b.shape
     k_pad = -(-k // 128) * 128
-    if b.dtype in _FP8_DTYPES and b.stride(0) == 1 and _packs_rows(b.t()):
-        return _pack_rows(b.t())
     if (b.is_cuda and b.dtype in (torch.float8_e5m2, torch.float8_e4m3fn) and b.is_contiguous()
             and n % 8 == 0 and n > 0 and k > 0 and b.data_ptr() % 8 == 0):
         out = torch.empty((k_pad // 16, n, 16), device=b.device, dtype=b.dtype)
         torch.ops.feather_ops.prepack_b.default(b, out)
         return out
+    if b.dtype in _FP8_DTYPES and b.stride(0) == 1 and _packs_rows(b.t()):
+        return _pack_rows(b.t())
     if k_pad != k:
         padded = torch.zeros((k_pad, n), device=b.device, dtype=b.dtype)
         padded[:k] = b

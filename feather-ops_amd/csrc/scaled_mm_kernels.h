@@ -344,19 +344,43 @@ __device__ __forceinline__ void store_wave_tiles(const Params& p, const f32x4 (&
 // Tile order: consecutive workgroup ids go to different XCDs, so give each XCD a contiguous run of tiles,
 // and walk tiles in groups of kGroupM tile rows so that the blocks resident on one XCD share A and B panels
 // in that XCD's L2.
-__device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m, int tiles_n, int& tm, int& tn) {
+__device__ __forceinline__ int xcd_run(int bid, int nblocks) {
     constexpr int kXcds = 8;
-    constexpr int kGroupM = 4;
     const int xcd = bid % kXcds;
     const int q = nblocks / kXcds;
     const int r = nblocks % kXcds;
-    const int t = xcd * q + (xcd < r ? xcd : r) + bid / kXcds;
+    return xcd * q + (xcd < r ? xcd : r) + bid / kXcds;
+}
+
+__device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m, int tiles_n, int& tm, int& tn) {
+    constexpr int kGroupM = 4;
+    const int t = xcd_run(bid, nblocks);
     const int group = t / (kGroupM * tiles_n);
     const int first_m = group * kGroupM;
     const int gm = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
     const int in = t - group * kGroupM * tiles_n;
     tm = first_m + in % gm;
     tn = in / gm;
+}
+
+// The streaming kernel's order. With several rows of tiles, each XCD gets a contiguous run of them, column by column: a
+// column's weight panel is read from memory once, into the L2 of the XCD that holds its rows. Row by row, a panel
+// reached up to 8 L2s unless the columns were a multiple of 8; there each column's rows share an XCD already, and the
+// interleaved columns measured up to 1.2x faster than runs. On 794 shapes and types (M 17-700; weights from HBM) the
+// heuristic's tiles ran 1.16x faster in geometric mean (0.84-2.1x) with runs everywhere.
+__device__ __forceinline__ void stream_tile_of_block(int bid, int n_tiles, int tiles_n, int& tm, int& tn) {
+    if (n_tiles == tiles_n) {
+        tm = 0;
+        tn = bid;
+    } else if (tiles_n % 8 == 0) {
+        tm = bid / tiles_n;
+        tn = bid - tm * tiles_n;
+    } else {
+        const int tiles_m = n_tiles / tiles_n;
+        const int t = xcd_run(bid, n_tiles);
+        tn = t / tiles_m;
+        tm = t - tn * tiles_m;
+    }
 }
 
 // ---- split-K join ------------------------------------------------------------------------------------------
@@ -1110,8 +1134,8 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     const int n_tiles = ((p.M + S::kBM - 1) / S::kBM) * tiles_n;
     const int split = kSplitK ? static_cast<int>(blockIdx.x) / n_tiles : 0;
     const int tile_id = static_cast<int>(blockIdx.x) - split * n_tiles;
-    const int tm = tile_id / tiles_n;
-    const int tn = tile_id % tiles_n;
+    int tm, tn;
+    stream_tile_of_block(tile_id, n_tiles, tiles_n, tm, tn);
     const int m0 = tm * S::kBM;
     const int n0 = tn * S::kBN + wave_n * 16 * RN;
 

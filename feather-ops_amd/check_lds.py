@@ -51,7 +51,8 @@ def expected_bytes(kernel: str, ints: list[int], bools: list[int] = ()) -> int:
     depth = 3 if k_slices * warps_n * repeat_n * (unroll_k // 4) <= 8 and repeat_m <= 2 else 2
     activations = k_slices * warps_n * depth * (unroll_k // 4) * repeat_m * 2048
     join = (k_slices if k_slices > 1 else 0) * warps_n * repeat_m * repeat_n * 64 * 16
-    return activations + join
+    # past 64 KiB the join lies over the activations (StreamShape::kJoinOverA)
+    return activations + join if activations + join <= 65536 or not join else max(activations, join)
 
 
 def compile_asm(combo: str) -> str:

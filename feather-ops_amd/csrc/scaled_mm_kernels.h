@@ -1105,7 +1105,13 @@ struct StreamShape {
     static constexpr int kABufBytes = kGroups * RM * kAFragBytes;
     static constexpr int kAWaveBytes = kDepth * kABufBytes;
     static constexpr int kALdsBytes = KS * WN * kAWaveBytes;
-    static constexpr int kLdsBytes = kALdsBytes + kRedBytes;
+    // Past 64 KiB (two blocks per CU) the join's buffer lies over the activations', which the block is done with by
+    // then (a barrier more): one to three blocks more per CU took 4-8% off such tiles at M 17-700, where the barrier
+    // costs the smaller ones 0.5%.
+    static constexpr bool kJoinOverA = kRedBytes > 0 && kALdsBytes + kRedBytes > 64 * 1024;
+    static constexpr int kRedBase = kJoinOverA ? 0 : kALdsBytes;
+    static constexpr int kLdsBytes = kJoinOverA ? (kALdsBytes > kRedBytes ? kALdsBytes : kRedBytes)
+                                                : kALdsBytes + kRedBytes;
     static constexpr int kLoadsPerFetch = kGroups * (2 * RM + RN);  // vector-memory ops of one fetch
     static_assert(U % 4 == 0, "an iteration is a whole number of 64-deep MFMA groups");
     static_assert(kThreads <= 1024, "block size");
@@ -1308,7 +1314,13 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
         // replays, bit-identical: C4 0.6% faster, the 32- and 64-row tiles 2-4%. Blocks narrower than 64 columns
         // (row segments of 32 or 64 bytes) keep the per-fragment join below, which measured 0.3-5.7% faster
         // there.
-        f32x4* red = reinterpret_cast<f32x4*>(lds + S::kALdsBytes);
+        f32x4* red = reinterpret_cast<f32x4*>(lds + S::kRedBase);
+        if constexpr (S::kJoinOverA) {
+            // this wave's direct loads (the last fetches' zeros too) have landed and its reads are done; then every wave's
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            __builtin_amdgcn_s_waitcnt(kLgkm0Imm);
+            __syncthreads();
+        }
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll
@@ -1360,7 +1372,13 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
         // Narrow blocks and split launches: the same parking, then the block's waves share the output
         // fragments, each adding a fragment's slices in slice order (and, split, joining it across workgroups)
         // and storing it; the fragment's bias loads are in flight during its join.
-        f32x4* red = reinterpret_cast<f32x4*>(lds + S::kALdsBytes);
+        f32x4* red = reinterpret_cast<f32x4*>(lds + S::kRedBase);
+        if constexpr (S::kJoinOverA) {
+            // this wave's direct loads (the last fetches' zeros too) have landed and its reads are done; then every wave's
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            __builtin_amdgcn_s_waitcnt(kLgkm0Imm);
+            __syncthreads();
+        }
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll

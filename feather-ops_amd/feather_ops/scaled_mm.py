@@ -650,12 +650,73 @@ def _tail_time(rows: int, N: int, K: int) -> float:
     return max(6.0, (3.0 + N * K / 5e6) * (1.0 if rows <= 16 else 1.35 if rows <= 32 else 1.8))
 
 
+# 16 < M <= 704 on the 16-row streaming tiles: taller tiles read the weight less often, and smaller ones fill the chip, by
+# a time model fitted on 267 shapes (M 17-700, N 512-16384, K 512-16384, weights from HBM) and both activation dtypes,
+# every tile timed on every shape. Microseconds of an unsplit launch of a tile: once, per block of a CU, per 64-deep
+# stage and 256 blocks, per stage with one block a CU, with two, with each of three or more, and per 5 MB of weight;
+# 5-9% in standard deviation (the 16-column tiles 13-15%). (fp16, bf16 activations.) Where a tile of _STREAM_REFINED is
+# predicted _STREAM_GAIN faster than the pick, it runs instead: 1.06x in geometric mean on the 534 shapes and types
+# (0.92-1.7x), against 1.08x for the best tile of each.
+_STREAM_TIME = {
+    (4, 1, 4, 1, 4, 0): ((2.89, 0.000, 0.015, 0.058, 0.105, 0.053, 0.500),
+                         (3.00, 0.000, 0.013, 0.065, 0.109, 0.054, 0.466)),
+    (4, 1, 4, 1, 2, 0): ((2.62, 0.000, 0.010, 0.033, 0.070, 0.036, 0.407),
+                         (2.76, 0.000, 0.009, 0.040, 0.076, 0.038, 0.394)),
+    (8, 1, 4, 1, 2, 0): ((2.71, 0.077, 0.012, 0.032, 0.066, 0.035, 0.392),
+                         (2.83, 0.088, 0.011, 0.033, 0.070, 0.036, 0.391)),
+    (4, 1, 4, 2, 2, 0): ((2.46, 0.187, 0.017, 0.053, 0.102, 0.052, 0.427),
+                         (2.54, 0.328, 0.014, 0.067, 0.118, 0.059, 0.359)),
+    (4, 1, 4, 2, 4, 0): ((2.91, 0.301, 0.021, 0.080, 0.141, 0.074, 0.408),
+                         (2.94, 0.452, 0.013, 0.099, 0.166, 0.084, 0.336)),
+    (8, 1, 4, 2, 4, 0): ((3.19, 0.597, 0.021, 0.078, 0.148, 0.071, 0.415),
+                         (3.21, 0.842, 0.019, 0.083, 0.156, 0.074, 0.391)),
+    (4, 1, 4, 3, 4, 0): ((3.48, 0.373, 0.016, 0.117, 0.193, 0.105, 0.308),
+                         (3.46, 0.582, 0.013, 0.142, 0.226, 0.115, 0.225)),
+    (4, 1, 4, 4, 4, 0): ((3.39, 0.778, 0.022, 0.143, 0.239, 0.127, 0.261),
+                         (3.31, 1.13, 0.016, 0.181, 0.288, 0.145, 0.166)),
+    (8, 1, 4, 1, 4, 0): ((2.90, 0.317, 0.013, 0.054, 0.105, 0.053, 0.473),
+                         (3.01, 0.336, 0.012, 0.055, 0.107, 0.053, 0.460)),
+    (4, 1, 8, 1, 4, 0): ((3.10, 0.151, 0.013, 0.052, 0.106, 0.055, 0.460),
+                         (3.33, 0.168, 0.012, 0.056, 0.111, 0.056, 0.426)),
+    (2, 2, 4, 2, 2, 0): ((2.87, 0.000, 0.015, 0.097, 0.210, 0.106, 0.467),
+                         (2.96, 0.121, 0.010, 0.139, 0.246, 0.127, 0.287)),
+    (4, 1, 4, 1, 1, 0): ((2.52, 0.000, 0.012, 0.026, 0.042, 0.023, 0.390),
+                         (2.69, 0.000, 0.011, 0.030, 0.046, 0.024, 0.357)),
+    (8, 1, 4, 1, 1, 0): ((2.19, 0.352, 0.012, 0.024, 0.041, 0.021, 0.332),
+                         (2.35, 0.386, 0.011, 0.025, 0.043, 0.022, 0.314)),
+}
+_STREAM_REFINED = tuple(_STREAM_TIME)[:8]
+_STREAM_REFINED_MAX_M = 704
+_STREAM_REFINED_MIN_SIDE = 512
+_STREAM_GAIN = 0.95
+
+
+def _stream_time(M: int, N: int, K: int, tile: tuple[int, ...], a_bf16: bool) -> float:
+    """Predicted microseconds of an unsplit streaming launch (_STREAM_TIME)."""
+    once, block, stage_blocks, one, two, more, weight = _STREAM_TIME[tile][a_bf16]
+    blocks, stages = _blocks(M, N, tile), -(-K // 64)
+    per_cu = -(-blocks // _CUS)
+    resident = one if per_cu == 1 else two if per_cu == 2 else more * per_cu
+    return once + block * per_cu + stages * (stage_blocks * blocks / _CUS + resident) + weight * N * K / 5e6
+
+
+def _refined(M: int, N: int, K: int, tile: tuple[int, int, int, int, int, int], splits: int,
+             a_bf16: bool) -> tuple[int, int, int, int, int, int]:
+    """The tile an unsplit streaming pick runs on."""
+    if (splits != 1 or tile not in _STREAM_TIME or not 16 < M <= _STREAM_REFINED_MAX_M
+            or min(N, K) < _STREAM_REFINED_MIN_SIDE):
+        return tile
+    best = min(_STREAM_REFINED, key=lambda t: _stream_time(M, N, K, t, a_bf16))
+    faster = _stream_time(M, N, K, best, a_bf16) <= _STREAM_GAIN * _stream_time(M, N, K, tile, a_bf16)
+    return best if faster else tile
+
+
 @functools.lru_cache(maxsize=4096)
 def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tuple[int, tuple[int, ...], int], ...], bool]:
     """The launches the auto path runs a shape as, ((rows, tile, splits), ...) from the first row on, and whether bf16
-    activations are widened first: `_auto_choice`'s single one, or two where the last few rows are better off alone."""
+    activations are widened first: `_auto_choice`'s single one (`_refined`), or two where the last few rows are better off alone."""
     tile, splits, widen = _auto_choice(M, N, K, a_dtype)
-    whole = ((M, tile, splits),), widen
+    whole = ((M, _refined(M, N, K, tile, splits, a_dtype == torch.bfloat16 and not widen), splits),), widen
     if M <= 256 or M % 128 == 0 or M % 128 > _TAIL_MAX_ROWS:
         return whole
     widen_us = max(_WIDEN_MIN_S, 4.0 * M * K / _WIDEN_BYTES_PER_S) * 1e6 if a_dtype == torch.bfloat16 else 0.0
@@ -679,8 +740,9 @@ def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tup
             continue
         time += _tail_time(M - rows, N, K) + widen_us
         if now >= _TAIL_MIN_GAIN * time and (best is None or time < best[0]):
-            tail = _auto_choice(M - rows, N, K, torch.float16)
-            best = time, ((rows, *main[:2]), (M - rows, *tail[:2]))
+            tile, splits, _ = _auto_choice(M - rows, N, K, torch.float16)
+            tail = _refined(M - rows, N, K, tile, splits, False), splits
+            best = time, ((rows, *main[:2]), (M - rows, *tail))
     return whole if best is None else (best[1], a_dtype == torch.bfloat16)
 
 

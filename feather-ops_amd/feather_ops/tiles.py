@@ -55,6 +55,11 @@ SCALED_MM_TILES = [
     (8, 2, 4, 1, 1, 0),  # 16 x 32, 8 K slices x 2 column waves
     (2, 2, 4, 2, 2, 0),  # 32 x 64
     (2, 2, 4, 4, 2, 0),  # 64 x 64
+    (4, 1, 4, 2, 2, 0),  # 32 x 32, 4 K slices
+    (4, 1, 4, 2, 4, 0),  # 32 x 64, 4 K slices
+    (8, 1, 4, 2, 4, 0),  # 32 x 64, 8 K slices
+    (4, 1, 4, 3, 4, 0),  # 48 x 64, 4 K slices
+    (4, 1, 4, 4, 4, 0),  # 64 x 64, 4 K slices
 ]
 
 # The tiles the gradient matmul runs with bf16 operands (`csrc/linear_backward.hip`): those the heuristic returns for

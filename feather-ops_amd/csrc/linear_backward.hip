@@ -6,7 +6,7 @@
 // The products are those of fp32 arithmetic, on the 16-bit MFMAs: an fp8 code is exact in fp16 and bf16, so a
 // 16-bit gradient times a code is exact in the fp32 accumulator. A per-tensor scale goes into the decode (its
 // power of two) and the epilogue. A per-column scale sits inside the sum: grad * scale is formed in fp32 and split
-// into three bf16 terms that sum to it exactly (split_columns_kernel), and the matmul runs over the three side by
+// into three bf16 terms that sum to it exactly (column_slab), and the matmul runs over the three side by
 // side, a contraction three times as long over three copies of the weight.
 //
 // Measured, forward and backward of 4096 rows through 3072 -> 12288 in bf16, one scale: 2732 us with torch's fp32
@@ -51,13 +51,12 @@ __device__ __forceinline__ uint32_t swizzled_unit(uint32_t k) {
     return (k & ~3u) | ((k ^ (k >> 4)) & 3u);
 }
 
-__global__ __launch_bounds__(kThreads) void transpose_prepacked_kernel(const uint8_t* b, uint8_t* out, uint32_t K,
-                                                                        uint32_t N, uint32_t n16, uint32_t copies,
-                                                                        bool e5m2, uint32_t k_tiles) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kTileChunks * kChunkPitch];
+__device__ __forceinline__ void transpose_tile(const uint8_t* b, uint8_t* out, uint32_t K, uint32_t N, uint32_t n16,
+                                               uint32_t copies, bool e5m2, uint32_t k_tiles, uint32_t tile,
+                                               uint8_t* lds) {
     const uint32_t t = threadIdx.x;
-    const uint32_t chunk0 = blockIdx.x % k_tiles * kTileChunks;
-    const uint32_t n0 = blockIdx.x / k_tiles * kTileCols;
+    const uint32_t chunk0 = tile % k_tiles * kTileChunks;
+    const uint32_t n0 = tile / k_tiles * kTileCols;
     const uint32_t chunks = K / 16u;
     const rsrc_t src = make_rsrc(b, chunks * N * 16u);
     const rsrc_t dst = make_rsrc(out, copies * n16 * K * 16u);
@@ -135,50 +134,6 @@ __device__ __forceinline__ void split3(float h, uint32_t (&t)[3]) {
     t[2] = finite ? __builtin_bit_cast(uint32_t, r2) >> 16 : 0u;
 }
 
-// g [M, N] times scale [N] -> out [M, 3 Nc] bf16, Nc = 16 * ceil(N / 16): the three terms of column n at n, Nc + n
-// and 2 Nc + n, zero past N. One work-item per 8 columns: 16 bytes in, 3 x 16 out. HBM-bound.
-template <bool kBf16>
-__global__ __launch_bounds__(kThreads) void split_columns_kernel(const uint16_t* g, const float* scale, uint16_t* out,
-                                                                  uint32_t M, uint32_t N, uint32_t nc) {
-    const uint32_t pieces = nc / 8u;
-    const uint32_t piece = blockIdx.x * kThreads + threadIdx.x;
-    const uint32_t row = piece / pieces;
-    const uint32_t col = piece % pieces * 8u;
-    if (row >= M) return;
-    const bool in = col < N;
-    const rsrc_t src = make_rsrc(g, M * N * 2u);
-    const rsrc_t scale_rsrc = make_rsrc(scale, N * 4u);
-    const rsrc_t dst = make_rsrc(out, M * nc * 6u);
-    const u32x4 v = buf_load16(src, in ? (row * N + col) * 2u : kOob);
-    const f32x4 s0 = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, in ? col * 4u : kOob));
-    const f32x4 s1 = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, in ? col * 4u + 16u : kOob));
-    u32x4 t[3];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const uint32_t pair = v[w];
-        float lo, hi;
-        if constexpr (kBf16) {
-            lo = __builtin_bit_cast(float, pair << 16);
-            hi = __builtin_bit_cast(float, pair & 0xffff0000u);
-        } else {
-            const half2v h = __builtin_bit_cast(half2v, pair);
-            lo = static_cast<float>(h[0]);
-            hi = static_cast<float>(h[1]);
-        }
-        const float sl = w < 2 ? s0[2 * w] : s1[2 * w - 4];
-        const float sh = w < 2 ? s0[2 * w + 1] : s1[2 * w - 3];
-        uint32_t tl[3], th[3];
-        split3(lo * sl, tl);
-        split3(hi * sh, th);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) t[i][w] = tl[i] | (th[i] << 16);
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < 3; ++i) {
-        __builtin_amdgcn_raw_buffer_store_b128(t[i], dst, static_cast<int>((row * 3u * nc + i * nc + col) * 2u), 0, 0);
-    }
-}
-
 // g [M, N] with N % 16 = 8 -> out [M, N + 8], zero in the new columns: the streaming kernel's rows are whole chunks.
 __global__ __launch_bounds__(kThreads) void pad_columns_kernel(const uint16_t* g, uint16_t* out, uint32_t M, uint32_t N) {
     const uint32_t pieces = N / 8u + 1u;
@@ -202,54 +157,112 @@ __device__ __forceinline__ uint16_t round16(float x) {
     return static_cast<uint16_t>(pack_out<kBf16>(x, x) & 0xffffu);
 }
 
-// Rows [y R, (y + 1) R) of 256 columns -> partial [y][N] fp32, or, alone (one slab of rows), `out`. HBM-bound: each
-// work-item keeps four 16-byte loads in flight (4096 x 12288: 17.4 us, 5.8 TB/s, against 272 for torch's sum). All sums
-// in fp32, in a fixed order.
-template <bool kBf16>
-__global__ __launch_bounds__(kThreads) void column_sums_kernel(const uint16_t* g, float* partial, uint16_t* out,
-                                                                uint32_t M, uint32_t N, uint32_t rows) {
-    __shared__ float red[kSumLanes][kSumCols];
-    const rsrc_t src = make_rsrc(g, M * N * 2u);
+struct Columns {
+    const uint16_t* g;      // [M, N]
+    float* partial;         // [slabs][N] sums of a slab's rows, or nullptr (no sums)
+    uint16_t* sums;         // [N], written here where there is a single slab
+    const float* scale;     // kSplit: [N]
+    uint16_t* terms;        // kSplit: [M, 3 nc] bf16, the terms of column n at n, nc + n and 2 nc + n, zero past N
+    uint32_t M, N, nc;      // nc = 16 * ceil(N / 16)
+    uint32_t rows, slabs;   // rows of a slab
+};
+
+// A slab's rows of 256 columns: their sums in fp32, in a fixed order (each work-item 8 columns of every eighth row, four
+// 16-byte loads in flight), and, kSplit, each element times its column's scale as three bf16 terms. HBM-bound (sums of
+// 4096 x 12288 alone: 17.4 us, 5.8 TB/s, against 272 for torch's sum).
+template <bool kBf16, bool kSplit>
+__device__ __forceinline__ void column_slab(const Columns& p, uint32_t tile, uint32_t slab, float (*red)[kSumCols]) {
+    const rsrc_t src = make_rsrc(p.g, p.M * p.N * 2u);
     const uint32_t lane = threadIdx.x / 32u;
     const uint32_t col_in = threadIdx.x % 32u * 8u;
-    const uint32_t col = blockIdx.x * kSumCols + col_in;
-    const uint32_t end = min(M, (blockIdx.y + 1) * rows);
+    const uint32_t col = tile * kSumCols + col_in;
+    const uint32_t end = min(p.M, (slab + 1) * p.rows);
+    float scale[8];
+    if constexpr (kSplit) {
+        const rsrc_t scale_rsrc = make_rsrc(p.scale, p.N * 4u);
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const f32x4 s = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, col < p.N ? col * 4u + 16u * h : kOob));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) scale[4 * h + i] = s[i];
+        }
+    }
     float sum[8] = {};
-    constexpr int kUnroll = 4;
-    for (uint32_t row = blockIdx.y * rows + lane; row < end; row += kUnroll * kSumLanes) {
+    constexpr uint32_t kUnroll = kSplit ? 4 : 8;
+    for (uint32_t row = slab * p.rows + lane; row < end; row += kUnroll * kSumLanes) {
         u32x4 v[kUnroll];
 #pragma unroll
         for (uint32_t i = 0; i < kUnroll; ++i) {
             const uint32_t r = row + i * kSumLanes;
-            v[i] = buf_load16(src, r < end && col < N ? (r * N + col) * 2u : kOob);
+            v[i] = buf_load16(src, r < end && col < p.N ? (r * p.N + col) * 2u : kOob);
         }
 #pragma unroll
-        for (int i = 0; i < kUnroll; ++i)
+        for (uint32_t i = 0; i < kUnroll; ++i) {
+            u32x4 t[3];
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 const uint32_t pair = v[i][w];
+                float lo, hi;
                 if constexpr (kBf16) {
-                    sum[2 * w] += __builtin_bit_cast(float, pair << 16);
-                    sum[2 * w + 1] += __builtin_bit_cast(float, pair & 0xffff0000u);
+                    lo = __builtin_bit_cast(float, pair << 16);
+                    hi = __builtin_bit_cast(float, pair & 0xffff0000u);
                 } else {
                     const half2v h = __builtin_bit_cast(half2v, pair);
-                    sum[2 * w] += static_cast<float>(h[0]);
-                    sum[2 * w + 1] += static_cast<float>(h[1]);
+                    lo = static_cast<float>(h[0]);
+                    hi = static_cast<float>(h[1]);
+                }
+                sum[2 * w] += lo;
+                sum[2 * w + 1] += hi;
+                if constexpr (kSplit) {
+                    uint32_t tl[3], th[3];
+                    split3(lo * scale[2 * w], tl);
+                    split3(hi * scale[2 * w + 1], th);
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) t[j][w] = tl[j] | (th[j] << 16);
                 }
             }
+            if constexpr (kSplit) {
+                const rsrc_t dst = make_rsrc(p.terms, p.M * p.nc * 6u);
+                const uint32_t r = row + i * kSumLanes;
+#pragma unroll
+                for (uint32_t j = 0; j < 3; ++j) {
+                    const uint32_t off = r < end && col < p.nc ? (r * 3u * p.nc + j * p.nc + col) * 2u : kOob;
+                    __builtin_amdgcn_raw_buffer_store_b128(t[j], dst, static_cast<int>(off), 0, 0);
+                }
+            }
+        }
     }
+    if (!p.partial) return;
 #pragma unroll
     for (int i = 0; i < 8; ++i) red[lane][col_in + i] = sum[i];
     __syncthreads();
-    const uint32_t c = blockIdx.x * kSumCols + threadIdx.x;
-    if (c >= N) return;
+    const uint32_t c = tile * kSumCols + threadIdx.x;
+    if (c >= p.N) return;
     float total = 0.f;
 #pragma unroll
     for (uint32_t i = 0; i < kSumLanes; ++i) total += red[i][threadIdx.x];
-    if (gridDim.y == 1) {
-        out[c] = round16<kBf16>(total);
+    if (p.slabs == 1) {
+        p.sums[c] = round16<kBf16>(total);
     } else {
-        partial[blockIdx.y * N + c] = total;
+        p.partial[slab * p.N + c] = total;
+    }
+}
+
+// What the matmul needs and the bias's gradient, in one launch: the first workgroups take a slab of the gradient's columns,
+// the last `transposes` a tile of the weight, side by side (1000 x 2560 -> 5120 with per-column scales: 15.8 us against
+// 10.2 + 8.0 + 5.1 in launches of their own).
+template <bool kBf16, bool kSplit>
+__global__ __launch_bounds__(kThreads) void prepare_kernel(const uint8_t* b, uint8_t* weight, uint32_t K, uint32_t n16,
+                                                            bool e5m2, uint32_t k_tiles, uint32_t transposes,
+                                                            Columns columns, uint32_t col_tiles) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kTileChunks * kChunkPitch];
+    static_assert(sizeof(lds) >= sizeof(float) * kSumLanes * kSumCols, "the sums' join fits");
+    const uint32_t slab_blocks = gridDim.x - transposes;
+    if (blockIdx.x >= slab_blocks) {
+        transpose_tile(b, weight, K, columns.N, n16, kSplit ? 3u : 1u, e5m2, k_tiles, blockIdx.x - slab_blocks, lds);
+    } else {
+        const uint32_t i = blockIdx.x;
+        column_slab<kBf16, kSplit>(columns, i % col_tiles, i / col_tiles, reinterpret_cast<float(*)[kSumCols]>(lds));
     }
 }
 
@@ -259,6 +272,7 @@ __global__ __launch_bounds__(kThreads) void column_sums_join_kernel(const float*
     const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
     if (c >= N) return;
     float total = 0.f;
+#pragma unroll 8
     for (uint32_t s = 0; s < slabs; ++s) total += partial[s * N + c];
     out[c] = round16<kBf16>(total);
 }
@@ -328,49 +342,53 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
     const Layout l = layout(M, N, K, per_column);
     uint8_t* const weight = static_cast<uint8_t*>(workspace);
     const uint32_t m = static_cast<uint32_t>(M), n = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
+    const bool pad = !prefetch && !per_column && N % 16 != 0;
+    const int64_t depth = pad ? N + 8 : l.depth;
+    const TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
+    uint16_t* const made = reinterpret_cast<uint16_t*>(weight + l.weight);
     if (grad_x) {
         if (!b_prepacked || !scale || !aligned16(b_prepacked) || !aligned16(grad_x)) return false;
         if (per_column && !aligned16(scale)) return false;
-        const TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
-        const bool pad = !prefetch && !per_column && N % 16 != 0;
-        const int64_t depth = pad ? N + 8 : l.depth;
-        uint16_t* const made = reinterpret_cast<uint16_t*>(weight + l.weight);
-        const uint16_t* const operand = per_column || pad ? made : grad;
         if (!grad_matmul_ok(tile, M, K, depth, bf16 || per_column, splits, split_workspace, split_workspace_bytes)) {
             return false;
         }
-        const uint32_t n16 = (n + 15) / 16;
-        const uint32_t k_tiles = (k + 16 * kTileChunks - 1) / (16 * kTileChunks);
-        const uint32_t n_tiles = (n + kTileCols - 1) / kTileCols;
-        hipLaunchKernelGGL(transpose_prepacked_kernel, dim3(k_tiles * n_tiles), dim3(kThreads), 0, stream, b_prepacked,
-                           weight, k, n, n16, per_column ? 3u : 1u, use_fp8_e5m2,
-                           k_tiles);
-        if (per_column) {
-            const uint32_t blocks = static_cast<uint32_t>((M * 2 * n16 + kThreads - 1) / kThreads);
-            hipLaunchKernelGGL(bf16 ? split_columns_kernel<true> : split_columns_kernel<false>, dim3(blocks),
-                               dim3(kThreads), 0, stream, grad, scale, made, m, n, 16 * n16);
-        } else if (pad) {
+    }
+    const bool split = grad_x && per_column;
+    const uint32_t n16 = (n + 15) / 16;
+    const uint32_t k_tiles = (k + 16 * kTileChunks - 1) / (16 * kTileChunks);
+    const uint32_t transposes = grad_x ? k_tiles * ((n + kTileCols - 1) / kTileCols) : 0;
+    const int64_t slabs = sum_slabs(M, N);
+    Columns columns{};
+    columns.g = grad;
+    columns.partial = grad_bias ? reinterpret_cast<float*>(weight + l.weight + l.terms) : nullptr;
+    columns.sums = grad_bias;
+    columns.scale = scale;
+    columns.terms = made;
+    columns.M = m;
+    columns.N = n;
+    columns.nc = 16 * n16;
+    columns.rows = static_cast<uint32_t>((M + slabs - 1) / slabs);
+    columns.slabs = (m + columns.rows - 1) / columns.rows;
+    const uint32_t col_tiles = (columns.nc + kSumCols - 1) / kSumCols;
+    const uint32_t slab_blocks = grad_bias || split ? col_tiles * columns.slabs : 0;
+    const auto prepare = split ? (bf16 ? prepare_kernel<true, true> : prepare_kernel<false, true>)
+                               : (bf16 ? prepare_kernel<true, false> : prepare_kernel<false, false>);
+    hipLaunchKernelGGL(prepare, dim3(transposes + slab_blocks), dim3(kThreads), 0, stream, b_prepacked, weight, k, n16,
+                       use_fp8_e5m2, k_tiles, transposes, columns, col_tiles);
+    if (grad_x) {
+        if (pad) {
             const uint32_t blocks = static_cast<uint32_t>((M * (N / 8 + 1) + kThreads - 1) / kThreads);
             hipLaunchKernelGGL(pad_columns_kernel, dim3(blocks), dim3(kThreads), 0, stream, grad, made, m, n);
         }
-        if (!launch_grad_matmul(tile, operand, weight, per_column ? nullptr : scale, grad_x, M, K, depth,
+        if (!launch_grad_matmul(tile, split || pad ? made : grad, weight, per_column ? nullptr : scale, grad_x, M, K, depth,
                                 use_fp8_e5m2, bf16 || per_column, bf16, splits, split_workspace, stream)) {
             return false;
         }
     }
-    if (grad_bias) {
-        float* const partial = reinterpret_cast<float*>(weight + l.weight + l.terms);
-        const int64_t slabs = sum_slabs(M, N);
-        const uint32_t rows = static_cast<uint32_t>((M + slabs - 1) / slabs);
-        const uint32_t used = (m + rows - 1) / rows;
-        hipLaunchKernelGGL(bf16 ? column_sums_kernel<true> : column_sums_kernel<false>,
-                           dim3((n + kSumCols - 1) / kSumCols, used), dim3(kThreads), 0, stream, grad, partial,
-                           grad_bias, m, n, rows);
-        if (used > 1) {
-            hipLaunchKernelGGL(bf16 ? column_sums_join_kernel<true> : column_sums_join_kernel<false>,
-                               dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, partial, grad_bias, n,
-                               used);
-        }
+    if (grad_bias && columns.slabs > 1) {
+        hipLaunchKernelGGL(bf16 ? column_sums_join_kernel<true> : column_sums_join_kernel<false>,
+                           dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, columns.partial, grad_bias, n,
+                           columns.slabs);
     }
     return true;
 }

@@ -700,23 +700,38 @@ def _stream_time(M: int, N: int, K: int, tile: tuple[int, ...], a_bf16: bool) ->
     return once + block * per_cu + stages * (stage_blocks * blocks / _CUS + resident) + weight * N * K / 5e6
 
 
+# 16 < M <= 32 and K >= 8192 (a decoder's down projection on a small batch): 32 x 64 tiles with 8 K slices read the weight
+# once where the 16-row picks read it twice, split along K to 200-256 workgroups of ranges 3072 deep or more: 1.28x in
+# geometric mean on the 14 such shapes and types of the sweeps (1.06-1.72x; 25 x 19072 -> 4736 35 -> 21 us; columns a
+# multiple of 512, whose re-reads stay in one XCD's L2, 1.0-1.2x). With fewer workgroups it loses (24 x 11008 -> 4096,
+# 192 of them: 0.89x).
+_STREAM_LONG_TILE = (8, 1, 4, 2, 4, 0)
+_STREAM_LONG_MAX_M = 32
+_STREAM_LONG_MIN_WORKGROUPS = 200
+
+
 def _refined(M: int, N: int, K: int, tile: tuple[int, int, int, int, int, int], splits: int,
-             a_bf16: bool) -> tuple[int, int, int, int, int, int]:
-    """The tile an unsplit streaming pick runs on."""
-    if (splits != 1 or tile not in _STREAM_TIME or not 16 < M <= _STREAM_REFINED_MAX_M
-            or min(N, K) < _STREAM_REFINED_MIN_SIDE):
-        return tile
-    best = min(_STREAM_REFINED, key=lambda t: _stream_time(M, N, K, t, a_bf16))
-    faster = _stream_time(M, N, K, best, a_bf16) <= _STREAM_GAIN * _stream_time(M, N, K, tile, a_bf16)
-    return best if faster else tile
+             a_bf16: bool) -> tuple[tuple[int, int, int, int, int, int], int]:
+    """(tile, splits) a streaming pick runs as past 16 rows."""
+    if not 16 < M <= _STREAM_REFINED_MAX_M or tile[5] != 0 or min(N, K) < _STREAM_REFINED_MIN_SIDE:
+        return tile, splits
+    if M <= _STREAM_LONG_MAX_M and K >= _STREAM_SPLIT_MIN_K:
+        blocks = _blocks(M, N, _STREAM_LONG_TILE)
+        most = min(8, _CUS // blocks, K // _STREAM_SPLIT_MIN_RANGE)
+        if most > 1 and blocks * most >= _STREAM_LONG_MIN_WORKGROUPS:
+            return _STREAM_LONG_TILE, most
+    if splits == 1 and tile in _STREAM_TIME:
+        best = min(_STREAM_REFINED, key=lambda t: _stream_time(M, N, K, t, a_bf16))
+        if _stream_time(M, N, K, best, a_bf16) <= _STREAM_GAIN * _stream_time(M, N, K, tile, a_bf16):
+            return best, 1
+    return tile, splits
 
 
-@functools.lru_cache(maxsize=4096)
 def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tuple[int, tuple[int, ...], int], ...], bool]:
     """The launches the auto path runs a shape as, ((rows, tile, splits), ...) from the first row on, and whether bf16
     activations are widened first: `_auto_choice`'s single one (`_refined`), or two where the last few rows are better off alone."""
     tile, splits, widen = _auto_choice(M, N, K, a_dtype)
-    whole = ((M, _refined(M, N, K, tile, splits, a_dtype == torch.bfloat16 and not widen), splits),), widen
+    whole = ((M, *_refined(M, N, K, tile, splits, a_dtype == torch.bfloat16 and not widen)),), widen
     if M <= 256 or M % 128 == 0 or M % 128 > _TAIL_MAX_ROWS:
         return whole
     widen_us = max(_WIDEN_MIN_S, 4.0 * M * K / _WIDEN_BYTES_PER_S) * 1e6 if a_dtype == torch.bfloat16 else 0.0
@@ -741,19 +756,19 @@ def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tup
         time += _tail_time(M - rows, N, K) + widen_us
         if now >= _TAIL_MIN_GAIN * time and (best is None or time < best[0]):
             tile, splits, _ = _auto_choice(M - rows, N, K, torch.float16)
-            tail = _refined(M - rows, N, K, tile, splits, False), splits
+            tail = _refined(M - rows, N, K, tile, splits, False)
             best = time, ((rows, *main[:2]), (M - rows, *tail))
     return whole if best is None else (best[1], a_dtype == torch.bfloat16)
 
 
 @functools.lru_cache(maxsize=4096)
-def _packed_tile(M: int, N: int, K: int, a_dtype: torch.dtype) -> int | None:
-    """The tile of a shape the auto path runs as one plain launch (unsplit, activations as given), its six numbers packed
-    into one for `feather_ops::scaled_mm_new`; None for the others."""
+def _auto_plan(M: int, N: int, K: int,
+               a_dtype: torch.dtype) -> tuple[tuple[tuple[int, tuple[int, ...], int], ...], bool, int | None]:
+    """`_auto_parts` and, where that is one plain launch (unsplit, activations as given), its tile's six numbers packed into
+    one for `feather_ops::scaled_mm_new` (else None): one lookup per call."""
     parts, widen = _auto_parts(M, N, K, a_dtype)
-    if widen or len(parts) > 1 or parts[0][2] > 1:
-        return None
-    return sum(field << 8 * i for i, field in enumerate(parts[0][1]))
+    plain = len(parts) == 1 and not widen and parts[0][2] == 1
+    return parts, widen, sum(field << 8 * i for i, field in enumerate(parts[0][1])) if plain else None
 
 
 # Split-K workspaces, one per (device, stream): the counter area at their start must be zero before a
@@ -857,14 +872,16 @@ def _widened(a: torch.Tensor) -> torch.Tensor:
 
 
 def _launch_auto(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bias: torch.Tensor | None,
-                 out: torch.Tensor) -> None:
-    """The heuristic's launch or launches."""
-    parts, widen = _auto_parts(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype)
-    if len(parts) == 1 or not _whole_rows(a) or not out.is_contiguous():
+                 out: torch.Tensor, plan: tuple | None = None) -> None:
+    """The heuristic's launch or launches (`plan`: their `_auto_plan`, where the caller has looked it up)."""
+    parts, widen = plan if plan is not None else _auto_plan(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype)[:2]
+    if len(parts) == 1:
+        _launch(a, b_prepacked, scale, bias, out, parts[0][1], parts[0][2], widen)
+        return
+    if not _whole_rows(a) or not out.is_contiguous():
         # activations the op would refuse go to it as they are, in one launch, so that it reports them
-        _, tile, splits = parts[0] if len(parts) == 1 else (0, *_auto_choice(a.shape[0], b_prepacked.shape[1],
-                                                                             a.shape[1], a.dtype)[:2])
-        _launch(a, b_prepacked, scale, bias, out, tile, splits, widen)
+        _launch(a, b_prepacked, scale, bias, out,
+                *_auto_choice(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype)[:2], widen)
         return
     if widen:
         a = _widened(a)
@@ -914,20 +931,20 @@ def scaled_mm_hip(
     """
     _lib.require_native()
     auto = tile is None and splits is None
-    if auto and (out_dtype is torch.bfloat16 or out_dtype is torch.float16) and not torch.compiler.is_compiling():
+    plan = None
+    if auto and not torch.compiler.is_compiling():
         shape = a.shape
-        packed = _packed_tile(shape[0], b_prepacked.shape[1], shape[1], a.dtype)
+        *plan, packed = _auto_plan(shape[0], b_prepacked.shape[1], shape[1], a.dtype)
         # operands that autograd follows take the ops that write into an output: it marks what an op returns
-        if packed is not None and not (a.requires_grad or b_prepacked.requires_grad
-                                       or (scale is not None and scale.requires_grad)
-                                       or (bias is not None and bias.requires_grad)):
+        if packed is not None and (out_dtype is torch.bfloat16 or out_dtype is torch.float16) and not (
+                a.requires_grad or b_prepacked.requires_grad or (scale is not None and scale.requires_grad)
+                or (bias is not None and bias.requires_grad)):
             return _scaled_mm_new(a, b_prepacked, scale, bias, out_dtype is torch.bfloat16, packed)
     out = torch.empty((a.shape[0], b_prepacked.shape[1]), device=a.device, dtype=out_dtype)
-    if auto:
-        if torch.compiler.is_compiling():
-            _scaled_mm_auto(a, b_prepacked, scale, bias, out)
-        else:
-            _launch_auto(a, b_prepacked, scale, bias, out)
+    if plan is not None:
+        _launch_auto(a, b_prepacked, scale, bias, out, plan)
+    elif auto:
+        _scaled_mm_auto(a, b_prepacked, scale, bias, out)
     else:
         if tile is None:
             tile = select_scaled_mm_config(a.shape[0], b_prepacked.shape[1], a.shape[1], a.dtype,

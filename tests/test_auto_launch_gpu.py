@@ -27,15 +27,16 @@ def _operands(m, n, k, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 1000, 2560), (77, 5120, 2560), (16, 14336, 4096), (0, 1000, 2560)])
 def test_same_bits_as_a_pinned_launch(fo, m, n, k, dtype):
-    from feather_ops.scaled_mm import _auto_parts, _packed_tile
+    from feather_ops.scaled_mm import _auto_plan
 
     a, b, scale = _operands(m, n, k, dtype)
-    assert _packed_tile(m, n, k, dtype) is not None
+    parts, _, packed = _auto_plan(m, n, k, dtype)
+    assert packed is not None
     for out_dtype in (torch.float16, torch.bfloat16):
         bias = torch.randn(n, device="cuda").to(out_dtype)
         for s in (None, scale, scale.expand(n).contiguous()):
             got = fo.scaled_mm_hip(a, b, s, bias, out_dtype)
-            want = fo.scaled_mm_hip(a, b, s, bias, out_dtype, tile=_auto_parts(m, n, k, dtype)[0][0][1])
+            want = fo.scaled_mm_hip(a, b, s, bias, out_dtype, tile=parts[0][1])
             assert got.shape == (m, n) and got.dtype == out_dtype and got.is_contiguous()
             assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from feather_ops.scaled_mm import _STREAM_REFINED, _STREAM_TIME, _auto_choice, _refined, _stream_time
-from feather_ops.tiles import SCALED_MM_TILES
+from feather_ops.tiles import SCALED_MM_TILES, split_workspace_bytes
 
 FP16, BF16 = torch.float16, torch.bfloat16
 
@@ -19,14 +19,19 @@ def test_rule_stays_in_its_range():
         m, n, k = int(2 ** rng.uniform(0, 11)), 8 * int(2 ** rng.uniform(4, 11)), 16 * int(2 ** rng.uniform(3, 10))
         for dtype in (FP16, BF16):
             tile, splits, widen = _auto_choice(m, n, k, dtype)
-            got = _refined(m, n, k, tile, splits, dtype == BF16 and not widen)
-            if got == tile:
+            got, got_splits = _refined(m, n, k, tile, splits, dtype == BF16 and not widen)
+            if (got, got_splits) == (tile, splits):
                 continue
-            changed.add(got)
-            assert got in _STREAM_REFINED and tile[5] == 0 and splits == 1
+            changed.add((got, got_splits > 1))
+            assert got in _STREAM_REFINED and tile[5] == 0
             assert 16 < m <= 704 and min(n, k) >= 512
-            assert _stream_time(m, n, k, got, dtype == BF16) < _stream_time(m, n, k, tile, dtype == BF16)
-    assert len(changed) >= 6
+            if got_splits > 1:
+                assert m <= 32 and 0 < split_workspace_bytes(m, n, k, got, got_splits) < 64 << 20
+                assert k // got_splits >= 3072 and 200 <= -(-n // 64) * got_splits <= 256
+            else:
+                assert splits == 1
+                assert _stream_time(m, n, k, got, dtype == BF16) < _stream_time(m, n, k, tile, dtype == BF16)
+    assert len(changed) >= 7 and any(split for _, split in changed)
 
 
 NEW = [(4, 1, 4, 2, 2, 0), (4, 1, 4, 2, 4, 0), (8, 1, 4, 2, 4, 0), (4, 1, 4, 3, 4, 0), (4, 1, 4, 4, 4, 0)]
@@ -67,7 +72,8 @@ def test_tall_tiles(tile, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [FP16, BF16])
-@pytest.mark.parametrize("m,n,k", [(77, 5120, 2560), (128, 3072, 3072), (300, 3072, 2560), (17, 4104, 528), (250, 2760, 1104)])
+@pytest.mark.parametrize("m,n,k", [(77, 5120, 2560), (128, 3072, 3072), (300, 3072, 2560), (17, 4104, 528), (250, 2760, 1104),
+                                   (25, 4736, 9216), (32, 5640, 12160)])
 def test_auto_path(m, n, k, dtype):
     import feather_ops
     from gpu_helpers import check_against_oracle

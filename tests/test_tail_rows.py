@@ -29,19 +29,19 @@ def test_parts_cover_the_rows_once():
     for _ in range(20000):
         m, n, k = int(2 ** rng.uniform(0, 14)), 8 * int(2 ** rng.uniform(0, 11)), 16 * int(2 ** rng.uniform(0, 10))
         for dtype in (FP16, BF16):
-            parts, widen = _auto_parts.__wrapped__(m, n, k, dtype)
+            parts, widen = _auto_parts(m, n, k, dtype)
             assert sum(rows for rows, _, _ in parts) == m
             if len(parts) == 1:
                 tile, splits, first = _auto_choice(m, n, k, dtype)
-                assert widen == first and parts[0][2] == splits
-                assert parts[0][1] == _refined(m, n, k, tile, splits, dtype == BF16 and not widen)
+                assert widen == first
+                assert parts[0][1:] == _refined(m, n, k, tile, splits, dtype == BF16 and not widen)
                 continue
             split += 1
             (head, tile, splits), (tail, *tail_pick) = parts
             assert head % 128 == 0 and splits == 1 and 0 < tail <= _TAIL_MAX_ROWS and m >= 320 - 64
             assert (tile, splits) == _auto_choice(head, n, k, FP16)[:2]
             tile, splits, _ = _auto_choice(tail, n, k, FP16)
-            assert tuple(tail_pick) == (_refined(tail, n, k, tile, splits, False), splits)
+            assert tuple(tail_pick) == _refined(tail, n, k, tile, splits, False)
     assert split > 50
     for m in (1, 77, 256, 512, 4096, 4224, 4096 + 100):
         assert len(_auto_parts(m, 4096, 4096, FP16)[0]) == 1

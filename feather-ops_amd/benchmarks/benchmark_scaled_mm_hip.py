@@ -4,7 +4,8 @@
 Same role and options as the reference's `bench/benchmark_scaled_mm_hip.py` (whole grid or groups or
 explicit cells, the heuristic against an explicit tile list, a square sweep): per cell it times
 `torch_mm` (torch's matmul on the already-dequantized bf16 weight: the optimistic control, which does
-not pay for dequantization), `auto` (the tile `select_scaled_mm_config` picks) and, with `--tiles`,
+not pay for dequantization), `auto` (the tile the auto path runs; where it gives the last
+rows a launch of their own, the one pick for all rows) and, with `--tiles`,
 every listed tile, interleaved (see protocol.py). It prints TFLOP/s per provider, the best tile and how
 far the heuristic's pick is from it, and with `--json` writes every measurement for refitting.
 
@@ -44,6 +45,7 @@ from benchmarks.cells import GROUPS, cells  # noqa: E402
 from benchmarks.protocol import measure, paired_speedup  # noqa: E402
 from feather_ops.scaled_mm import (  # noqa: E402
     _auto_choice,
+    _auto_parts,
     prepack_b_for_scaled_mm,
     select_scaled_mm_config,
     select_scaled_mm_splits,
@@ -109,6 +111,9 @@ def run_cell(m: int, n: int, k: int, tiles, args) -> dict:
     picked = tuple(select_scaled_mm_config(m, n, k, a_dtype, fp8, out_dtype))
     picked_splits = select_scaled_mm_splits(m, n, k, picked, a_dtype)
     wide_tile, wide_splits, widen = _auto_choice(m, n, k, a_dtype)
+    parts, _ = _auto_parts(m, n, k, a_dtype)
+    if len(parts) == 1 and not widen:   # what the auto path runs the pick as (past 16 rows, streaming)
+        _, picked, picked_splits = parts[0]
     # bf16 activations: time the widening pass + fp16-activation pick against the in-place bf16 pick where the
     # heuristic widens first, or on every cell with --widen-all (the data its rule is fitted on)
     compare_widen = a_dtype == torch.bfloat16 and (widen or args.widen_all)

@@ -970,8 +970,10 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
         out = torch.empty((k_pad // 16, n, 16), device=b.device, dtype=b.dtype)
         torch.ops.feather_ops.prepack_b.default(b, out)
         return out
-    if b.dtype in _FP8_DTYPES and b.stride(0) == 1 and _packs_rows(b.t()):
-        return _pack_rows(b.t())
+    if b.dtype in _FP8_DTYPES and b.stride(0) == 1:
+        w = b.t()
+        if _packs_rows(w):
+            return _pack_rows(w)
     if k_pad != k:
         padded = torch.zeros((k_pad, n), device=b.device, dtype=b.dtype)
         padded[:k] = b
@@ -983,11 +985,13 @@ def _packs_rows(w: torch.Tensor) -> bool:
     """Whether the row-packing kernels take `w` [N, K]: an fp8 (to lay out), bf16, fp16 or fp32 (to quantize) weight on
     the GPU, its rows whole 16-byte units and its buffers under 2 GiB; a plain tensor, outside tracing and
     transforms, whose copies autograd does not follow."""
-    return (w.is_cuda and w.dim() == 2 and w.dtype in _PACKED_DTYPES and w.is_contiguous() and w.numel() > 0
-            and w.shape[1] % 16 == 0 and type(w) in (torch.Tensor, torch.nn.Parameter)
+    if not w.is_cuda or w.dim() != 2 or not w.is_contiguous() or type(w) not in (torch.Tensor, torch.nn.Parameter):
+        return False
+    n, k = w.shape
+    bytes_per = _PACKED_BYTES.get(w.dtype)
+    return (bytes_per is not None and k % 16 == 0 and 0 < n * (k + 127 & -128) * bytes_per < 1 << 31
             and not torch.compiler.is_compiling() and not torch._C._functorch.is_functorch_wrapped_tensor(w)
-            and w.data_ptr() % 16 == 0 and w.shape[0] * (-(-w.shape[1] // 128) * 128) * w.element_size() < 1 << 31
-            and not (w.requires_grad and torch.is_grad_enabled()))
+            and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled()))
 
 
 def quantize_and_pack(w: torch.Tensor, fp8_dtype: torch.dtype,
@@ -1005,7 +1009,7 @@ def quantize_and_pack(w: torch.Tensor, fp8_dtype: torch.dtype,
 
 
 _FP8_DTYPES = (torch.float8_e5m2, torch.float8_e4m3fn)
-_PACKED_DTYPES = _FP8_DTYPES + (torch.bfloat16, torch.float16, torch.float32)
+_PACKED_BYTES = {torch.float8_e5m2: 1, torch.float8_e4m3fn: 1, torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
 
 
 def _pack_rows(w: torch.Tensor) -> torch.Tensor:

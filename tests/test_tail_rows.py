@@ -93,6 +93,16 @@ def test_graph_replays():
 
 
 @pytest.mark.gpu
+def test_operands_that_require_grad():
+    import feather_ops
+
+    a, b, scale, bias = _inputs(1281, 5960, 5248, FP16, True)
+    want = feather_ops.scaled_mm_hip(a, b, scale, bias, FP16)
+    out = feather_ops.scaled_mm_hip(a.requires_grad_(), b, scale, bias, FP16)
+    assert not out.requires_grad and torch.equal(out, want)
+
+
+@pytest.mark.gpu
 def test_refused_operands_are_refused_as_before():
     import feather_ops
 

@@ -9,10 +9,10 @@
 // into three bf16 terms that sum to it exactly (column_slab), and the matmul runs over the three side by
 // side, a contraction three times as long over three copies of the weight.
 //
-// Measured, forward and backward of 4096 rows through 3072 -> 12288 in bf16, one scale: 2732 us with torch's fp32
-// operations (1.9 ms its fp32 matmul, 0.27 ms the column sums, 0.2 ms dequantizing the weight), 435 us here: the
+// Measured, forward and backward of 4096 rows through 3072 -> 12288 in bf16, one scale: 2744 us with torch's fp32
+// operations (2.0 ms its fp32 matmul, 0.27 ms the column sums, 0.17 ms dequantizing the weight), 436 us here: the
 // matmul's 309 GFLOP take 215-238 us (1.3-1.4 PFLOP/s, the rate of the forward's). 1000 rows through 2560 -> 5120 in
-// fp16 with per-column scales: 322 us, 158 us here (the three-term matmul 78 us, 1.0 PFLOP/s).
+// fp16 with per-column scales: 334 us of kernels, 128 here (the three-term matmul 74 us, 1.06 PFLOP/s).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -59,6 +59,15 @@ def test_every_tile_is_computed_once(rows, columns):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("columns", [2, 3, 5, 8])
+@pytest.mark.parametrize("rows", [2, 9, 16, 27, 42])
+def test_every_tile_of_a_tall_problem_is_computed_once(rows, columns):
+    """Both sides of N = 4/3 M, where the runs turn from columns to rows; rows not a multiple of the 8 XCDs."""
+    _check(16 * rows - 3, 64 * columns - 8, 272, (4, 1, 4, 1, 4, 0), FP16)
+    _check(16 * rows, 64 * columns, 1040, (4, 1, 4, 1, 4, 0), BF16, splits=2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("tile", NEW + [(2, 2, 4, 4, 2, 0), (8, 1, 8, 1, 4, 0)])
 def test_tall_tiles(tile, dtype):

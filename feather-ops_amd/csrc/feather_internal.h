@@ -24,7 +24,8 @@ extern "C" {
  *
  * Sums are fp32: products of 16-bit gradients and fp8 codes are exact in them, and a per-column scale is multiplied
  * into the gradient in fp32 without loss afterwards. Requires N % 8 == 0, K % 16 == 0 and 16-byte aligned pointers;
- * returns false (nothing enqueued) otherwise, and for a tile, a split count or a workspace that does not fit.
+ * returns false (nothing enqueued) otherwise, and for a tile or split count that feather_linear_backward_split_bytes
+ * refuses, or a workspace that is too small.
  */
 bool feather_linear_backward(const uint16_t* grad, const uint8_t* b_prepacked, const float* scale, uint16_t* grad_x,
                              uint16_t* grad_bias, int64_t M, int64_t N, int64_t K, bool per_column, bool use_fp8_e5m2,
@@ -37,6 +38,14 @@ int64_t feather_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K,
 
 /* The inputs (contraction length) of feather_linear_backward's matmul: what its tile and splits are chosen for. */
 int64_t feather_linear_backward_depth(int64_t N, bool per_column);
+
+/*
+ * Bytes of split_workspace that feather_linear_backward needs with this tile and split count (0 for splits = 1), for
+ * gradients of either type; -1 where it refuses them. Host only: what a caller asks before it leaves another path.
+ */
+int64_t feather_linear_backward_split_bytes(int64_t M, int64_t N, int64_t K, bool per_column, int block_warps_m,
+                                            int block_warps_n, int unroll_k, int repeat_m, int repeat_n, bool prefetch,
+                                            int splits);
 
 /*
  * w [N, K] row-major -> out [K_pad/16][N][16], zero-padded to K_pad = ceil(K / 128) * 128: the layout of

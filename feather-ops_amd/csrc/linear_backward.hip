@@ -134,7 +134,7 @@ __device__ __forceinline__ void split3(float h, uint32_t (&t)[3]) {
     t[2] = finite ? __builtin_bit_cast(uint32_t, r2) >> 16 : 0u;
 }
 
-// g [M, N] with N % 16 = 8 -> out [M, N + 8], zero in the new columns: the streaming kernel's rows are whole chunks.
+// g [M, N] with N % 16 = 8 -> out [M, N + 8], zero in the new columns (pads_columns).
 __global__ __launch_bounds__(kThreads) void pad_columns_kernel(const uint16_t* g, uint16_t* out, uint32_t M, uint32_t N) {
     const uint32_t pieces = N / 8u + 1u;
     const uint32_t piece = blockIdx.x * kThreads + threadIdx.x;
@@ -290,7 +290,7 @@ constexpr int64_t align256(int64_t n) {
 }
 
 struct Layout {
-    int64_t depth;         // the matmul's contraction: N, or 3 * 16 * ceil(N / 16) with per-column scales
+    int64_t depth;         // the matmul's contraction: N (16 for 8), or 3 * 16 * ceil(N / 16) with per-column scales
     int64_t weight;        // bytes of the transposed weight, at 0
     int64_t terms;         // of the split gradient, or of a padded one (N % 16 = 8), after it
     int64_t sums;          // of the column sums' partials, after that
@@ -300,11 +300,22 @@ struct Layout {
 Layout layout(int64_t M, int64_t N, int64_t K, bool per_column) {
     const int64_t n16 = (N + 15) / 16;
     Layout l{};
-    l.depth = per_column ? 3 * 16 * n16 : N;
+    l.depth = per_column ? 3 * 16 * n16 : std::max<int64_t>(N, 16);
     l.weight = align256((l.depth + 127) / 128 * 8 * K * 16);
     l.terms = per_column ? align256(M * l.depth * 2) : N % 16 ? align256(M * 16 * n16 * 2) : 0;
     l.sums = align256(sum_slabs(M, N) * N * 4);
     return l;
+}
+
+// The matmul takes the gradient padded to whole chunks: on streaming tiles, whose rows are whole chunks, and on every
+// tile where one chunk is all there is.
+bool pads_columns(int64_t N, bool per_column, bool prefetch) {
+    return !per_column && N % 16 != 0 && (!prefetch || N < 16);
+}
+
+// The contraction of the launch itself: the padded columns included.
+int64_t launch_depth(int64_t N, bool per_column, bool prefetch) {
+    return pads_columns(N, per_column, prefetch) ? N + 8 : layout(1, N, 16, per_column).depth;
 }
 
 bool aligned16(const void* p) {
@@ -316,6 +327,15 @@ bool aligned16(const void* p) {
 
 extern "C" int64_t feather_linear_backward_depth(const int64_t N, const bool per_column) {
     return feather::layout(1, N, 16, per_column).depth;
+}
+
+extern "C" int64_t feather_linear_backward_split_bytes(const int64_t M, const int64_t N, const int64_t K,
+                                                       const bool per_column, const int block_warps_m,
+                                                       const int block_warps_n, const int unroll_k, const int repeat_m,
+                                                       const int repeat_n, const bool prefetch, const int splits) {
+    if (feather_linear_backward_workspace_bytes(M, N, K, per_column) < 0) return -1;
+    const feather::TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
+    return feather::grad_matmul_split_bytes(tile, M, K, feather::launch_depth(N, per_column, prefetch), true, splits);
 }
 
 extern "C" int64_t feather_linear_backward_workspace_bytes(const int64_t M, const int64_t N, const int64_t K,
@@ -342,16 +362,16 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
     const Layout l = layout(M, N, K, per_column);
     uint8_t* const weight = static_cast<uint8_t*>(workspace);
     const uint32_t m = static_cast<uint32_t>(M), n = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
-    const bool pad = !prefetch && !per_column && N % 16 != 0;
-    const int64_t depth = pad ? N + 8 : l.depth;
+    const bool pad = pads_columns(N, per_column, prefetch);
+    const int64_t depth = launch_depth(N, per_column, prefetch);
     const TileQuery tile{block_warps_m, block_warps_n, unroll_k, repeat_m, repeat_n, prefetch};
     uint16_t* const made = reinterpret_cast<uint16_t*>(weight + l.weight);
     if (grad_x) {
         if (!b_prepacked || !scale || !aligned16(b_prepacked) || !aligned16(grad_x)) return false;
         if (per_column && !aligned16(scale)) return false;
-        if (!grad_matmul_ok(tile, M, K, depth, bf16 || per_column, splits, split_workspace, split_workspace_bytes)) {
-            return false;
-        }
+        const int64_t split_bytes = grad_matmul_split_bytes(tile, M, K, depth, bf16 || per_column, splits);
+        if (split_bytes < 0 || split_bytes > split_workspace_bytes) return false;
+        if (splits > 1 && (!split_workspace || (reinterpret_cast<uintptr_t>(split_workspace) & 255u))) return false;
     }
     const bool split = grad_x && per_column;
     const uint32_t n16 = (n + 15) / 16;

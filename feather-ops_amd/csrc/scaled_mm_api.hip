@@ -203,13 +203,11 @@ Params make_params(const uint16_t* a, const uint8_t* b_prepacked, const float* s
 
 }  // namespace
 
-bool grad_matmul_ok(const TileQuery& t, int64_t M, int64_t K, int64_t depth, bool operand_bf16, int splits,
-                    const void* split_workspace, int64_t split_workspace_bytes) {
-    if (depth < 16 || depth % (t.prefetch ? 8 : 16) != 0 || depth * M * 2 > kMaxBufferBytes) return false;
-    const SplitLayout l =
-        split_layout(M, K, depth, t.warps_m, t.warps_n, t.unroll_k, t.repeat_m, t.repeat_n, t.prefetch, splits);
-    if (l.total_bytes < 0 || (operand_bf16 && !is_grad_tile(t))) return false;
-    return splits == 1 || (split_workspace && aligned(split_workspace, 256) && split_workspace_bytes >= l.total_bytes);
+int64_t grad_matmul_split_bytes(const TileQuery& t, int64_t M, int64_t K, int64_t depth, bool operand_bf16, int splits) {
+    if (depth < 16 || depth % (t.prefetch ? 8 : 16) != 0 || depth * M * 2 > kMaxBufferBytes) return -1;
+    if (operand_bf16 && !is_grad_tile(t)) return -1;
+    return split_layout(M, K, depth, t.warps_m, t.warps_n, t.unroll_k, t.repeat_m, t.repeat_n, t.prefetch, splits)
+        .total_bytes;
 }
 
 bool launch_grad_matmul(const TileQuery& t, const uint16_t* operand, const uint8_t* b, const float* scale,

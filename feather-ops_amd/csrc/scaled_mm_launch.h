@@ -37,9 +37,10 @@ bool launch_combo_121(const TileQuery&, const Params&, hipStream_t);
 
 // grad_x [M, K] = operand [M, depth] @ b [depth/16, K, 16] * scale (one value; none: 1), the gradient matmul of
 // linear_backward.hip: depth a multiple of 8 (streaming tiles: 16), the operand bf16 (operand_bf16) or fp16, the output bf16 or fp16 (fp16
-// operands: fp16). `grad_matmul_ok` says on the host whether the tile, the splits and their workspace fit.
-bool grad_matmul_ok(const TileQuery& tile, int64_t M, int64_t K, int64_t depth, bool operand_bf16, int splits,
-                    const void* split_workspace, int64_t split_workspace_bytes);
+// operands: fp16). `grad_matmul_split_bytes` says on the host what workspace the splits need, 256-byte aligned (0: none),
+// or -1 where the tile or the splits do not fit.
+int64_t grad_matmul_split_bytes(const TileQuery& tile, int64_t M, int64_t K, int64_t depth, bool operand_bf16,
+                                int splits);
 bool launch_grad_matmul(const TileQuery& tile, const uint16_t* operand, const uint8_t* b, const float* scale,
                         uint16_t* grad_x, int64_t M, int64_t K, int64_t depth, bool use_fp8_e5m2, bool operand_bf16,
                         bool out_bf16, int splits, void* split_workspace, hipStream_t stream);

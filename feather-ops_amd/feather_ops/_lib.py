@@ -43,6 +43,9 @@ def c_library() -> ctypes.CDLL:
         lib.feather_linear_backward_workspace_bytes.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool]
         lib.feather_linear_backward_depth.restype = ctypes.c_int64
         lib.feather_linear_backward_depth.argtypes = [ctypes.c_int64, ctypes.c_bool]
+        lib.feather_linear_backward_split_bytes.restype = ctypes.c_int64
+        lib.feather_linear_backward_split_bytes.argtypes = ([ctypes.c_int64] * 3 + [ctypes.c_bool] + [ctypes.c_int] * 5 +
+                                                            [ctypes.c_bool, ctypes.c_int])
         _c_library = lib
     return _c_library
 

@@ -11,7 +11,7 @@ import functools
 import torch
 
 from . import _lib
-from .scaled_mm import _auto_choice, _split_workspace, _workspace_bytes
+from .scaled_mm import _auto_choice, _split_workspace
 
 # Layers of fewer products than this keep torch's fp32 matmul: launches and host work bound both there (60 rows of 256 ->
 # 192: forward and backward 143 us a pass against 88), and callers of such layers compare gradients with that product
@@ -22,8 +22,8 @@ _MIN_PRODUCTS = 1 << 22
 @functools.lru_cache(maxsize=4096)
 def backward_plan(M: int, N: int, K: int, per_column: bool) -> tuple[tuple[int, ...], int, int, int] | None:
     """(tile, splits, split workspace bytes, workspace bytes) of a layer of N outputs and K inputs on M rows, or None
-    where the layer stays with `composite`: small ones (_MIN_PRODUCTS), and those whose buffers would pass 2 GiB (or whose
-    sizes are outside the forward's contract)."""
+    where the layer stays with `composite`: small ones (_MIN_PRODUCTS), and what the library's own check refuses: buffers
+    past 2 GiB, sizes outside the forward's contract."""
     if M * N * K < _MIN_PRODUCTS:
         return None
     lib = _lib.c_library()
@@ -32,7 +32,7 @@ def backward_plan(M: int, N: int, K: int, per_column: bool) -> tuple[tuple[int, 
         return None
     depth = lib.feather_linear_backward_depth(N, per_column)
     tile, splits, _ = _auto_choice(M, K, depth, torch.float16)
-    split_bytes = _workspace_bytes(M, K, depth, tile, splits) if splits > 1 else 0
+    split_bytes = lib.feather_linear_backward_split_bytes(M, N, K, per_column, *tile, splits)
     return (tile, splits, split_bytes, nbytes) if split_bytes >= 0 else None
 
 

@@ -6,6 +6,7 @@ import random
 import pytest
 import torch
 
+from feather_ops import _lib
 from feather_ops import linear_backward as lb
 from feather_ops import prepack_transpose
 from feather_ops.tiles import GRAD_TILES, SCALED_MM_TILES, split_workspace_bytes
@@ -27,11 +28,23 @@ def test_grad_tiles_cover_the_picks():
                 continue
             tile, splits, split_bytes, nbytes = plan
             assert tile in GRAD_TILES, (m, n, k, tile)
-            depth = 48 * -(-n // 16) if column else n
+            depth = 48 * -(-n // 16) if column else max(n, 16)
             assert splits == 1 or split_bytes == split_workspace_bytes(m, k, depth, tile, splits)
             assert nbytes >= -(-depth // 128) * 128 * k + (2 * m * depth if column else 0)
             seen.add(tile)
     assert seen == set(GRAD_TILES)
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 8, 4096), (4096, 8, 4096), (4112, 8, 3072), (64, 8, 16384), (512, 24, 4096)])
+def test_plans_pass_the_librarys_check(m, n, k):
+    """A router's or a gate's few outputs: one chunk of depth, the least any kernel takes."""
+    lib = _lib.c_library()
+    for column in (False, True):
+        tile, splits, split_bytes, _ = lb.backward_plan(m, n, k, column)
+        assert lib.feather_linear_backward_split_bytes(m, n, k, column, *tile, splits) == split_bytes >= 0
+    assert lib.feather_linear_backward_split_bytes(m, n, k, False, 3, 3, 3, 3, 3, True, 1) == -1
+    assert lib.feather_linear_backward_split_bytes(m, n, k, False, *tile, 99) == -1
+    assert lib.feather_linear_backward_split_bytes(m, n + 4, k, False, *tile, 1) == -1
 
 
 def test_plan_refuses_buffers_past_2_gib():

@@ -56,10 +56,10 @@ def _check(lb, grad, wq, scale):
 
 
 # (m, n, k): a row; a depth of one and a half chunks; tails in every axis; N % 16 = 8 on the ring, wide and streaming
-# kernels; each kernel's split launch; the wide tiles whole and ragged.
-SHAPES = [(1, 1000, 1024), (3, 24, 32), (77, 1000, 2560), (1000, 5120, 2560), (300, 1000, 1008), (513, 2568, 1040),
-          (257, 4096, 4096), (20, 16384, 1024), (40, 5120, 12288), (4096, 3080, 3072), (4096, 4096, 4096),
-          (1040, 6144, 1536)]
+# kernels; each kernel's split launch; the wide tiles whole and ragged; 8 outputs on the ring kernel's tiles.
+SHAPES = [(1, 1000, 1024), (3, 24, 32), (512, 8, 4096), (4096, 8, 4096), (77, 1000, 2560), (1000, 5120, 2560),
+          (300, 1000, 1008), (513, 2568, 1040), (257, 4096, 4096), (20, 16384, 1024), (40, 5120, 12288),
+          (4096, 3080, 3072), (4096, 4096, 4096), (1040, 6144, 1536)]
 
 
 @pytest.mark.parametrize("column", [False, True])

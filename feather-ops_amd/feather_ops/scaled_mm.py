@@ -895,6 +895,22 @@ _lib.load()
 _scaled_mm_new = torch.ops.feather_ops.scaled_mm_new.default
 
 
+@torch.library.register_fake("feather_ops::scaled_mm_new")
+def _(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bias: torch.Tensor | None, out_bf16: bool,
+      tile: int) -> torch.Tensor:
+    # Fake tensors only (shape propagation, make_fx): like the ops that write into an output, none of them for the
+    # meta device itself.
+    if a.device.type == "meta":
+        raise NotImplementedError("feather_ops::scaled_mm_new: attempted to run this operator with Meta tensors")
+    return a.new_empty((a.shape[0], b_prepacked.shape[1]), dtype=torch.bfloat16 if out_bf16 else torch.float16)
+
+
+@torch.library.register_vmap("feather_ops::scaled_mm_new")
+def _(info, in_dims, *args):
+    # as the ops that write into an output do; vmap's loop would take some shapes (one plain launch) and refuse others
+    raise RuntimeError("Batching rule not implemented for feather_ops::scaled_mm_new")
+
+
 @custom_op("feather_ops::scaled_mm_auto", mutates_args=("out",))
 def _scaled_mm_auto(
     a: torch.Tensor,

@@ -1,0 +1,62 @@
+"""Shape propagation and make_fx over the auto path, with fake CUDA tensors on the CPU: each kind of unsplit launch gives
+the output's shape and a program that runs alone."""
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+
+import feather_ops
+from feather_ops import scaled_mm as impl
+
+FP16, BF16 = torch.float16, torch.bfloat16
+SHAPES = [(0, 64, 128), (1, 1000, 2560), (77, 1000, 2560), (4096, 12288, 3072)]
+
+
+def _operands(m, n, k, dtype, device="cuda"):
+    return (torch.empty((m, k), dtype=dtype, device=device),
+            torch.empty((-(-k // 128) * 8, n, 16), dtype=torch.float8_e5m2, device=device),
+            torch.empty((), device=device))
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_shape_propagation(m, n, k, dtype):
+    with FakeTensorMode():
+        a, b, scale = _operands(m, n, k, dtype)
+        for out_dtype in (FP16, BF16):
+            out = feather_ops.scaled_mm_hip(a, b, scale, None, out_dtype)
+            assert out.shape == (m, n) and out.dtype == out_dtype and out.device == a.device and out.is_contiguous()
+
+
+@pytest.mark.parametrize("mode", ["fake", "symbolic"])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_make_fx(m, n, k, mode):
+    from torch.fx.experimental.symbolic_shapes import ShapeEnv
+
+    with FakeTensorMode(shape_env=ShapeEnv()):
+        operands = _operands(m, n, k, FP16)
+    graph = make_fx(lambda a, b, s: feather_ops.scaled_mm_hip(a, b, s, None, FP16), tracing_mode=mode)(*operands).graph
+    nodes = [node for node in graph.nodes if node.op != "placeholder"]
+    assert not any(node.op == "get_attr" for node in nodes)
+    launches = [node for node in nodes if "feather_ops" in str(node.target)]
+    assert len(launches) == len(impl._auto_plan(m, n, k, FP16)[0])
+
+
+def test_relabelled_linear_without_gradients():
+    with FakeTensorMode():
+        lin = torch.nn.Linear(2560, 1000, device="cuda", dtype=BF16).requires_grad_(False)
+        feather_ops.to_scaled_mm_linear(lin)
+        assert lin(torch.empty((2, 5, 2560), device="cuda", dtype=BF16)).shape == (2, 5, 1000)
+
+
+def test_what_the_two_step_call_refuses():
+    with pytest.raises(NotImplementedError, match="Meta"):
+        feather_ops.scaled_mm_hip(*_operands(16, 1000, 2560, FP16, "meta"), None, FP16)
+    with pytest.raises(NotImplementedError, match="CPU"):
+        feather_ops.scaled_mm_hip(*_operands(16, 1000, 2560, FP16, "cpu"), None, FP16)
+    with FakeTensorMode():
+        _, b, scale = _operands(16, 1000, 2560, FP16)
+        with pytest.raises(RuntimeError, match="Batching rule not implemented"):
+            torch.vmap(lambda a: feather_ops.scaled_mm_hip(a, b, scale, None, FP16))(
+                torch.empty((3, 16, 2560), dtype=FP16, device="cuda"))

@@ -19,6 +19,7 @@ Pass `tile=` to pin it, which is what the benchmark sweeps and the tests do.
 import functools
 
 import torch
+from torch._subclasses.fake_tensor import FakeTensor
 from torch.library import custom_op
 
 from . import _lib
@@ -860,7 +861,10 @@ def _launch(
         if nbytes < 0:
             raise RuntimeError(
                 f"split-K needs an instantiated tile and 1 <= splits <= the K units, got {tile}, {splits}")
-        ws = _split_workspace(a.device, nbytes)
+        if isinstance(a, FakeTensor):  # made in the traced program, not in the cache that real calls read
+            ws = torch.zeros(nbytes, dtype=torch.uint8, device=a.device)
+        else:
+            ws = _split_workspace(a.device, nbytes)
     torch.ops.feather_ops.scaled_mm_splitk.default(a, b_prepacked, scale, bias, out, ws, splits, *tile)
 
 

@@ -1,5 +1,5 @@
-"""Shape propagation and make_fx over the auto path, with fake CUDA tensors on the CPU: each kind of unsplit launch gives
-the output's shape and a program that runs alone."""
+"""Shape propagation and make_fx over the auto path, with fake CUDA tensors on the CPU: each kind of launch (plain, split,
+widened first, last rows apart) gives the output's shape and a program that runs alone, and leaves nothing behind."""
 
 import pytest
 import torch
@@ -10,7 +10,7 @@ import feather_ops
 from feather_ops import scaled_mm as impl
 
 FP16, BF16 = torch.float16, torch.bfloat16
-SHAPES = [(0, 64, 128), (1, 1000, 2560), (77, 1000, 2560), (4096, 12288, 3072)]
+SHAPES = [(0, 64, 128), (1, 1000, 2560), (77, 1000, 2560), (40, 5120, 12288), (4096, 12288, 3072), (4112, 4096, 12288)]
 
 
 def _operands(m, n, k, dtype, device="cuda"):
@@ -19,14 +19,26 @@ def _operands(m, n, k, dtype, device="cuda"):
             torch.empty((), device=device))
 
 
+def test_shapes_cover_the_launches():
+    kinds = set()
+    for m, n, k in SHAPES:
+        for dtype in (FP16, BF16):
+            parts, widen, packed = impl._auto_plan(m, n, k, dtype)
+            kinds |= {"plain" if packed is not None else "widened" if widen else "split" if len(parts) == 1 else "parts"}
+            kinds |= {"parts"} if len(parts) > 1 else set()
+    assert kinds == {"plain", "split", "widened", "parts"}
+
+
 @pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("m,n,k", SHAPES)
 def test_shape_propagation(m, n, k, dtype):
+    before = dict(impl._split_workspaces)
     with FakeTensorMode():
         a, b, scale = _operands(m, n, k, dtype)
         for out_dtype in (FP16, BF16):
             out = feather_ops.scaled_mm_hip(a, b, scale, None, out_dtype)
             assert out.shape == (m, n) and out.dtype == out_dtype and out.device == a.device and out.is_contiguous()
+    assert impl._split_workspaces == before
 
 
 @pytest.mark.parametrize("mode", ["fake", "symbolic"])
@@ -39,6 +51,9 @@ def test_make_fx(m, n, k, mode):
     graph = make_fx(lambda a, b, s: feather_ops.scaled_mm_hip(a, b, s, None, FP16), tracing_mode=mode)(*operands).graph
     nodes = [node for node in graph.nodes if node.op != "placeholder"]
     assert not any(node.op == "get_attr" for node in nodes)
+    for node in nodes:
+        if node.target is torch.ops.feather_ops.scaled_mm_splitk.default:
+            assert node.args[5].target is torch.ops.aten.zeros.default   # its counters start at zero
     launches = [node for node in nodes if "feather_ops" in str(node.target)]
     assert len(launches) == len(impl._auto_plan(m, n, k, FP16)[0])
 

@@ -583,6 +583,8 @@ def widen_first(M: int, N: int, K: int, tile: tuple[int, ...], splits: int) -> b
     on wide weights, the 128 x 128 and 64 x 128 tiles at long K (4096x4608x4608 1.08x, 4608x4096x16384 1.09x,
     1072x5120x8192 1.11x) and, with
     M <= 64, the 64 x 64 tile on big weights (32x25600x5120 1.19x, 32x8192x28672 split 4 ways 1.22x)."""
+    if K < 16:   # the op refuses it
+        return False
     kernel_s = 2.0 * M * N * K / _WIDEN_FLOPS
     if M <= _WIDEN_DEEP_MAX_M and tuple(tile) == _TILE_RING_64x64:
         lead = _WIDEN_LEAD_DEEP_64x64
@@ -733,7 +735,7 @@ def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tup
     activations are widened first: `_auto_choice`'s single one (`_refined`), or two where the last few rows are better off alone."""
     tile, splits, widen = _auto_choice(M, N, K, a_dtype)
     whole = ((M, *_refined(M, N, K, tile, splits, a_dtype == torch.bfloat16 and not widen)),), widen
-    if M <= 256 or M % 128 == 0 or M % 128 > _TAIL_MAX_ROWS:
+    if M <= 256 or M % 128 == 0 or M % 128 > _TAIL_MAX_ROWS or K < 16:
         return whole
     widen_us = max(_WIDEN_MIN_S, 4.0 * M * K / _WIDEN_BYTES_PER_S) * 1e6 if a_dtype == torch.bfloat16 else 0.0
     if a_dtype == torch.bfloat16 and not widen:

@@ -47,6 +47,13 @@ def test_parts_cover_the_rows_once():
         assert len(_auto_parts(m, 4096, 4096, FP16)[0]) == 1
 
 
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("m,n,k", [(320, 64, 0), (4112, 4096, 0), (300, 0, 64), (0, 64, 64), (4112, 4096, 8)])
+def test_empty_sides_are_one_launch(m, n, k, dtype):
+    """The op itself answers them: an empty result, or its refusal of K."""
+    assert _auto_parts(m, n, k, dtype) == (((m, *_auto_choice(m, n, k, dtype)[:2]),), _auto_choice(m, n, k, dtype)[2])
+
+
 def _inputs(m, n, k, dtype, column):
     import feather_ops
 

@@ -12,6 +12,7 @@ from collections.abc import Callable
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 # (original class, mixin) -> the relabelled class, so every relabel of the same pair yields one type object.
 _CLASS_CACHE: dict[tuple[type, type], type] = {}
@@ -129,9 +130,10 @@ def _linear_backward(ctx, grad: torch.Tensor):
     weight_fp8, weight_scale = ctx.saved_tensors
     k = ctx.x_shape[-1]
     need_x, need_bias = ctx.needs_input_grad[0], ctx.bias_dtype is not None and ctx.needs_input_grad[3]
-    # A gradient that is itself differentiated (create_graph) or batched by a transform (vmap, grad of grad) takes
-    # torch's operations, which have rules for both.
-    if (torch.is_grad_enabled() and grad.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(grad):
+    # A gradient that is itself differentiated (create_graph, or a tangent of forward mode) or batched by a transform
+    # (vmap, grad of grad) takes torch's operations, which have rules for all of them.
+    if ((torch.is_grad_enabled() and grad.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(grad)
+            or forward_ad.unpack_dual(grad).tangent is not None):
         grad_x, grad_bias = composite(grad, weight_fp8, weight_scale, k)
     else:
         grad_x, grad_bias = linear_backward(grad, weight_fp8, weight_scale, k, need_x, need_bias)

@@ -65,3 +65,23 @@ def test_operands_off_the_gpu_take_torch(column):
     assert torch.equal(bias, grad.reshape(10, 24).float().sum(0).to(torch.bfloat16))
     none_x, none_b = lb.linear_backward(grad, prepack_transpose(wq), scale, 48, False, False)
     assert none_x.numel() == none_b.numel() == 0
+
+
+def test_tangents_of_gradients():
+    """Forward mode over the backward (a Hessian-vector product): the gradient's tangent reaches both results."""
+    import types
+
+    from torch.autograd import forward_ad
+
+    from feather_ops.modules import _linear_backward
+
+    torch.manual_seed(0)
+    packed, scale = prepack_transpose(torch.randn(24, 48).to(torch.float8_e5m2)), torch.rand(24)
+    ctx = types.SimpleNamespace(saved_tensors=(packed, scale), x_shape=(2, 5, 48), x_dtype=torch.float16,
+                                bias_dtype=torch.float16, needs_input_grad=(True, False, False, True))
+    grad, tangent = torch.randn(2, 2, 5, 24).to(torch.float16)
+    want = [x for x in _linear_backward(ctx, tangent) if x is not None]
+    with forward_ad.dual_level():
+        got = [x for x in _linear_backward(ctx, forward_ad.make_dual(grad, tangent)) if x is not None]
+        got = [forward_ad.unpack_dual(x).tangent for x in got]
+    assert len(got) == 2 and all(torch.equal(a, b) for a, b in zip(got, want))

@@ -22,8 +22,9 @@ extern "C" {
  *                (sized for that matmul); otherwise it is ignored.
  *   workspace    feather_linear_backward_workspace_bytes(...) bytes, 16-byte aligned, of any content.
  *
- * Sums are fp32: products of 16-bit gradients and fp8 codes are exact in them, and a per-column scale is multiplied
- * into the gradient in fp32 without loss afterwards. Requires N % 8 == 0, K % 16 == 0 and 16-byte aligned pointers;
+ * Sums are fp32: products of 16-bit gradients and fp8 codes are exact in them. A per-column scale is multiplied into the
+ * gradient in fp32, and the matmul takes the product in three bf16 terms: all of it, but for what lies under 2^-133 times
+ * the largest scale's code (fp16 gradients: where |gradient * scale| < 2^-110, far below what fp16 results hold). Requires N % 8 == 0, K % 16 == 0 and 16-byte aligned pointers;
  * returns false (nothing enqueued) otherwise, and for a tile or split count that feather_linear_backward_split_bytes
  * refuses, or a workspace that is too small.
  */

@@ -6,8 +6,10 @@
 // The products are those of fp32 arithmetic, on the 16-bit MFMAs: an fp8 code is exact in fp16 and bf16, so a
 // 16-bit gradient times a code is exact in the fp32 accumulator. A per-tensor scale goes into the decode (its
 // power of two) and the epilogue. A per-column scale sits inside the sum: grad * scale is formed in fp32 and split
-// into three bf16 terms that sum to it exactly (column_slab), and the matmul runs over the three side by
-// side, a contraction three times as long over three copies of the weight.
+// into three bf16 terms that sum to it (column_slab), and the matmul runs over the three side by side, a contraction
+// three times as long over three copies of the weight. bf16 gradients reach sizes whose products with a scale (2^-19
+// of the weight's size in e5m2) have no three terms left above bf16's least value, so there the scales are taken times
+// the power of two that brings the largest near 1 (scale_up), and the weight's decode divides by it.
 //
 // Measured, forward and backward of 4096 rows through 3072 -> 12288 in bf16, one scale: 2744 us with torch's fp32
 // operations (2.0 ms its fp32 matmul, 0.27 ms the column sums, 0.17 ms dequantizing the weight), 436 us here: the
@@ -120,8 +122,9 @@ __device__ __forceinline__ void transpose_tile(const uint8_t* b, uint8_t* out, u
 
 // ---- per-column scales -----------------------------------------------------------------------------------------
 
-// h (24 significant bits) = t[0] + t[1] + t[2], bf16 bits each, by truncation: exact, and t[0] never overflows. Of
-// inf and NaN the first term carries everything.
+// h (24 significant bits) = t[0] + t[1] + t[2], bf16 bits each, by truncation: exact from |h| = 2^-110 on (below, what
+// falls under bf16's least value, 2^-133, is lost), and t[0] never overflows. Of inf and NaN the first term carries
+// everything.
 __device__ __forceinline__ void split3(float h, uint32_t (&t)[3]) {
     const uint32_t bits = __builtin_bit_cast(uint32_t, h);
     const bool finite = (bits & 0x7f800000u) != 0x7f800000u;
@@ -132,6 +135,30 @@ __device__ __forceinline__ void split3(float h, uint32_t (&t)[3]) {
     const float r2 = r1 - __builtin_bit_cast(float, bits1 & 0xffff0000u);
     t[1] = finite ? bits1 >> 16 : 0u;
     t[2] = finite ? __builtin_bit_cast(uint32_t, r2) >> 16 : 0u;
+}
+
+// The power of two, 1 to 2^100, that takes the largest finite |scale| of N into [0.5, 1), or as near below as it goes; 1
+// where that is 0.5 or more. |gradient * scale| then stays under |gradient|, so nothing overflows that did not, and what
+// split3 loses of a product is under 2^-132 times the largest weight, about the least step of a bf16 result. Every
+// workgroup reads all the scales (64 KiB at N = 16384, from L2).
+__device__ __forceinline__ float scale_up(const float* scale, uint32_t N, uint32_t (&top)[kThreads / kWave]) {
+    const rsrc_t src = make_rsrc(scale, N * 4u);
+    uint32_t most = 0;
+    for (uint32_t n = threadIdx.x * 4u; n < N; n += kThreads * 4u) {
+        const u32x4 v = buf_load16(src, n * 4u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t magnitude = v[i] & 0x7fffffffu;
+            most = max(most, magnitude < 0x7f800000u ? magnitude : 0u);
+        }
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(most, d)));
+    if (threadIdx.x % kWave == 0) top[threadIdx.x / kWave] = most;
+    __syncthreads();
+    const uint32_t exponent = max(max(top[0], top[1]), max(top[2], top[3])) >> 23;
+    const uint32_t up = exponent >= 126u ? 0u : min(126u - exponent, 100u);
+    return __builtin_bit_cast(float, (127u + up) << 23);
 }
 
 // g [M, N] with N % 16 = 8 -> out [M, N + 8], zero in the new columns (pads_columns).
@@ -162,6 +189,7 @@ struct Columns {
     float* partial;         // [slabs][N] sums of a slab's rows, or nullptr (no sums)
     uint16_t* sums;         // [N], written here where there is a single slab
     const float* scale;     // kSplit: [N]
+    float* unscale;         // kSplit of bf16 gradients: 1 / scale_up goes here, for the matmul
     uint16_t* terms;        // kSplit: [M, 3 nc] bf16, the terms of column n at n, nc + n and 2 nc + n, zero past N
     uint32_t M, N, nc;      // nc = 16 * ceil(N / 16)
     uint32_t rows, slabs;   // rows of a slab
@@ -171,7 +199,8 @@ struct Columns {
 // 16-byte loads in flight), and, kSplit, each element times its column's scale as three bf16 terms. HBM-bound (sums of
 // 4096 x 12288 alone: 17.4 us, 5.8 TB/s, against 272 for torch's sum).
 template <bool kBf16, bool kSplit>
-__device__ __forceinline__ void column_slab(const Columns& p, uint32_t tile, uint32_t slab, float (*red)[kSumCols]) {
+__device__ __forceinline__ void column_slab(const Columns& p, uint32_t tile, uint32_t slab, float (*red)[kSumCols],
+                                            uint32_t (&top)[kThreads / kWave]) {
     const rsrc_t src = make_rsrc(p.g, p.M * p.N * 2u);
     const uint32_t lane = threadIdx.x / 32u;
     const uint32_t col_in = threadIdx.x % 32u * 8u;
@@ -185,6 +214,12 @@ __device__ __forceinline__ void column_slab(const Columns& p, uint32_t tile, uin
             const f32x4 s = __builtin_bit_cast(f32x4, buf_load16(scale_rsrc, col < p.N ? col * 4u + 16u * h : kOob));
 #pragma unroll
             for (int i = 0; i < 4; ++i) scale[4 * h + i] = s[i];
+        }
+        if constexpr (kBf16) {
+            const float up = scale_up(p.scale, p.N, top);
+            if (blockIdx.x == 0 && threadIdx.x == 0) *p.unscale = 1.0f / up;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) scale[i] *= up;
         }
     }
     float sum[8] = {};
@@ -257,12 +292,14 @@ __global__ __launch_bounds__(kThreads) void prepare_kernel(const uint8_t* b, uin
                                                             Columns columns, uint32_t col_tiles) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kTileChunks * kChunkPitch];
     static_assert(sizeof(lds) >= sizeof(float) * kSumLanes * kSumCols, "the sums' join fits");
+    __shared__ uint32_t top[kThreads / kWave];
     const uint32_t slab_blocks = gridDim.x - transposes;
     if (blockIdx.x >= slab_blocks) {
         transpose_tile(b, weight, K, columns.N, n16, kSplit ? 3u : 1u, e5m2, k_tiles, blockIdx.x - slab_blocks, lds);
     } else {
         const uint32_t i = blockIdx.x;
-        column_slab<kBf16, kSplit>(columns, i % col_tiles, i / col_tiles, reinterpret_cast<float(*)[kSumCols]>(lds));
+        column_slab<kBf16, kSplit>(columns, i % col_tiles, i / col_tiles, reinterpret_cast<float(*)[kSumCols]>(lds),
+                                   top);
     }
 }
 
@@ -294,7 +331,8 @@ struct Layout {
     int64_t weight;        // bytes of the transposed weight, at 0
     int64_t terms;         // of the split gradient, or of a padded one (N % 16 = 8), after it
     int64_t sums;          // of the column sums' partials, after that
-    int64_t total() const { return weight + terms + sums; }
+    int64_t unscale;       // of one float, last
+    int64_t total() const { return weight + terms + sums + unscale; }
 };
 
 Layout layout(int64_t M, int64_t N, int64_t K, bool per_column) {
@@ -304,6 +342,7 @@ Layout layout(int64_t M, int64_t N, int64_t K, bool per_column) {
     l.weight = align256((l.depth + 127) / 128 * 8 * K * 16);
     l.terms = per_column ? align256(M * l.depth * 2) : N % 16 ? align256(M * 16 * n16 * 2) : 0;
     l.sums = align256(sum_slabs(M, N) * N * 4);
+    l.unscale = per_column ? align256(4) : 0;
     return l;
 }
 
@@ -383,6 +422,7 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
     columns.partial = grad_bias ? reinterpret_cast<float*>(weight + l.weight + l.terms) : nullptr;
     columns.sums = grad_bias;
     columns.scale = scale;
+    columns.unscale = reinterpret_cast<float*>(weight + l.weight + l.terms + l.sums);
     columns.terms = made;
     columns.M = m;
     columns.N = n;
@@ -400,8 +440,9 @@ extern "C" bool feather_linear_backward(const uint16_t* const grad, const uint8_
             const uint32_t blocks = static_cast<uint32_t>((M * (N / 8 + 1) + kThreads - 1) / kThreads);
             hipLaunchKernelGGL(pad_columns_kernel, dim3(blocks), dim3(kThreads), 0, stream, grad, made, m, n);
         }
-        if (!launch_grad_matmul(tile, split || pad ? made : grad, weight, per_column ? nullptr : scale, grad_x, M, K, depth,
-                                use_fp8_e5m2, bf16 || per_column, bf16, splits, split_workspace, stream)) {
+        const float* const rest = !per_column ? scale : bf16 ? columns.unscale : nullptr;
+        if (!launch_grad_matmul(tile, split || pad ? made : grad, weight, rest, grad_x, M, K, depth, use_fp8_e5m2,
+                                bf16 || per_column, bf16, splits, split_workspace, stream)) {
             return false;
         }
     }

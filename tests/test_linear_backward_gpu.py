@@ -41,7 +41,7 @@ def _operands(m, n, k, dtype, fp8, column, size=1e-2, seed=0):
     return grad, wq, scale
 
 
-def _check(lb, grad, wq, scale):
+def _check(lb, grad, wq, scale, lost=0.0):
     from feather_ops import prepack_transpose
 
     n, k = wq.shape
@@ -51,7 +51,7 @@ def _check(lb, grad, wq, scale):
     half, least = (2.0**-8, 2.0**-134) if grad.dtype == BF16 else (2.0**-11, 2.0**-25)
     for got, want, terms, depth in ((x, grad.double() @ w, grad.double().abs() @ w.abs(), 3 * n),
                                     (bias, grad.double().sum(0), grad.double().abs().sum(0), grad.shape[0])):
-        bound = half * want.abs() + least + (depth + 2) * 2.0**-24 * terms
+        bound = half * want.abs() + least + (depth + 2) * 2.0**-24 * terms + (lost if got is x else 0.0)
         assert ((got.double() - want).abs() <= bound).all()
 
 
@@ -80,6 +80,27 @@ def test_fp16_subnormal_gradients(lb, every_size, column):
 def test_scales_of_any_size_and_sign(lb, every_size, column, factor):
     grad, wq, scale = _operands(70, 264, 272, BF16, E4M3, column)
     _check(lb, grad, wq, scale * factor)
+
+
+@pytest.mark.parametrize("size", [1e-30, 1e-33, 1e-35, 1e-36, 1e-37])
+@pytest.mark.parametrize("fp8", [E5M2, E4M3])
+@pytest.mark.parametrize("column", [False, True])
+def test_bf16_gradients_near_the_least_value(lb, every_size, column, fp8, size):
+    """bf16's least normal value is 1.2e-38. At 1e-37 with per-column scales the gradient's last term ends at bf16's least
+    step, 2^-133, which meets the codes over the power of two of the scales."""
+    grad, wq, scale = _operands(70, 264, 272, BF16, fp8, column, size=size)
+    lost = 0.0
+    if column and size < 1e-36:
+        lost = 2.0**-133 * wq.double().abs().sum(0) * 2.0**(scale.max().log2().floor() + 1).double()
+    _check(lb, grad, wq, scale, lost)
+
+
+@pytest.mark.parametrize("size", [1e-2, 1e-33, 2.0**120])
+def test_scales_far_apart(lb, every_size, size):
+    """One power of two serves all the columns of a layer, and the largest decides it."""
+    grad, wq, scale = _operands(70, 264, 272, BF16, E5M2, True, size=size)
+    powers = torch.arange(264, device="cuda") % 33 - 32
+    _check(lb, grad, wq, scale * 2.0**powers)
 
 
 def test_bf16_gradients_near_the_largest_value(lb, every_size):

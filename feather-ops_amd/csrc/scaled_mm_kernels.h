@@ -55,6 +55,16 @@ constexpr uint32_t kOob = 0x80000000u;
 // Buffer resource word 3 for gfx9-family raw (untyped, stride 0) buffers.
 constexpr int kRsrcFlags = 0x00020000;
 
+// The streaming kernel's order of tiles (stream_order): workgroups take lines of `length` tiles, rows of tiles (kByRow) or
+// columns, one line after the other.
+struct TileOrder {
+    uint32_t length;
+    uint32_t inverse;           // min(2^32 - 1, floor(2^32 / length))
+    uint32_t tiles;             // of the launch (under 2^24: M N < 2^30), and the flags
+    static constexpr uint32_t kRuns = 1u << 30;    // contiguous runs of tiles on each XCD; otherwise workgroup id order
+    static constexpr uint32_t kByRow = 1u << 31;
+};
+
 struct Params {
     const uint16_t* a;          // [M, K] fp16 or bf16 bits, row-major
     const uint8_t* b;           // [kb_total, N, 16] fp8 codes
@@ -62,6 +72,7 @@ struct Params {
     const uint16_t* bias;       // [N] in the output dtype, or nullptr
     uint16_t* c;                // [M, N] output bits, row-major
     int32_t M, N, K;
+    TileOrder order;            // streaming kernel: set by the launcher
     int32_t kb_total;           // b_prepacked.shape[0]
     int32_t col_scale;          // scale holds one value per output column (16-byte aligned)
     // Split-K (ring kernel only): each output tile's 64-deep stages are cut into `splits` contiguous
@@ -365,31 +376,41 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m,
 
 // The streaming kernel's order. With several rows of tiles, each XCD gets a contiguous run of them, column by column: a
 // column's weight panel is read from memory once, into the L2 of the XCD that holds its rows. Row by row, a panel
-// reached up to 8 L2s unless the columns were a multiple of 8; there each column's rows share an XCD already, and the
-// interleaved columns measured up to 1.2x faster than runs. On 794 shapes and types (M 17-700; weights from HBM) the
-// heuristic's tiles ran 1.16x faster in geometric mean (0.84-2.1x) with runs everywhere.
+// reaches 8 / gcd(8, columns) L2s: one where the columns are a multiple of 8, where row by row stays (up to 1.2x faster than
+// runs). On 562 shapes and types (M 17-700; weights from HBM) the heuristic's tiles ran 1.16x as fast in geometric mean
+// (0.85-2.1x) with runs off the multiples of 8 as row by row.
 // Tall problems (N < 4/3 M, activations at least 1.5 times the weights) get runs row by row instead: each XCD reads its own
 // rows once and the small weights from its L2, where a run of columns reads all the activations again in every column.
 // On 91 such shapes and types of 7 us and more it is 1.16x faster than column runs in geometric mean (0.98-1.64x, the more
 // the fewer columns: 1640 x 2464 -> 736 bf16 18.4 -> 15.1 us, 606 x 7104 -> 232 fp16 15.2 -> 9.2); the gain ends
 // between N = 1.3 M (1.00x) and 1.9 M (0.87x at 891 x 3728 -> 1680).
-__device__ __forceinline__ void stream_tile_of_block(int bid, int n_tiles, int tiles_n, bool tall, int& tm, int& tn) {
-    if (n_tiles == tiles_n) {
-        tm = 0;
-        tn = bid;
-    } else if (tall) {
-        const int t = xcd_run(bid, n_tiles);
-        tm = t / tiles_n;
-        tn = t - tm * tiles_n;
-    } else if (tiles_n % 8 == 0) {
-        tm = bid / tiles_n;
-        tn = bid - tm * tiles_n;
-    } else {
-        const int tiles_m = n_tiles / tiles_n;
-        const int t = xcd_run(bid, n_tiles);
-        tn = t / tiles_m;
-        tm = t - tn * tiles_m;
+// The host picks the order and prepares the division: worked out in the kernel ahead of its first load, it cost every block
+// of a call with several rows of tiles 0.1 us (31 x 560 -> 320 2.39 us against 2.27).
+inline TileOrder stream_order(int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n) {
+    TileOrder o{};
+    const bool tall = 3 * N < 4 * M;
+    const bool runs = tiles_m > 1 && (tall || tiles_n % 8 != 0);
+    const bool by_row = !runs || tall;
+    o.length = static_cast<uint32_t>(by_row ? tiles_n : tiles_m);
+    o.inverse = o.length == 1 ? ~0u : static_cast<uint32_t>((uint64_t{1} << 32) / o.length);
+    o.tiles = static_cast<uint32_t>(tiles_m * tiles_n) | (runs ? TileOrder::kRuns : 0u) | (by_row ? TileOrder::kByRow : 0u);
+    return o;
+}
+
+__device__ __forceinline__ void stream_tile_of_block(uint32_t bid, const TileOrder& o, int& tm, int& tn) {
+    const uint32_t tiles = o.tiles & (TileOrder::kRuns - 1);
+    const uint32_t xcd = bid % 8;
+    const uint32_t t = o.tiles & TileOrder::kRuns ? xcd * (tiles / 8) + min(xcd, tiles % 8) + bid / 8 : bid;
+    // t / length: the rounded-down inverse gives the quotient or one less, t being under 2^32
+    uint32_t line = __umulhi(t, o.inverse);
+    uint32_t place = t - line * o.length;
+    if (place >= o.length) {
+        ++line;
+        place -= o.length;
     }
+    const bool by_row = o.tiles & TileOrder::kByRow;
+    tm = static_cast<int>(by_row ? line : place);
+    tn = static_cast<int>(by_row ? place : line);
 }
 
 // ---- split-K join ------------------------------------------------------------------------------------------
@@ -1150,7 +1171,7 @@ __global__ __launch_bounds__(kWave * KS * WN) void stream_kernel(const Params p)
     const int split = kSplitK ? static_cast<int>(blockIdx.x) / n_tiles : 0;
     const int tile_id = static_cast<int>(blockIdx.x) - split * n_tiles;
     int tm, tn;
-    stream_tile_of_block(tile_id, n_tiles, tiles_n, 3 * p.N < 4 * p.M, tm, tn);
+    stream_tile_of_block(tile_id, p.order, tm, tn);
     const int m0 = tm * S::kBM;
     const int n0 = tn * S::kBN + wave_n * 16 * RN;
 

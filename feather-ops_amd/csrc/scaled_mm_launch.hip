@@ -124,11 +124,14 @@ bool try_tile(const TileQuery& t, const Params& p, hipStream_t stream) {
         }
     } else {
         using S = StreamShape<WM, WN, U, RM, RN>;
-        const int64_t tiles = ((p.M + S::kBM - 1) / S::kBM) * static_cast<int64_t>((p.N + S::kBN - 1) / S::kBN);
+        const int64_t tiles_m = (p.M + S::kBM - 1) / S::kBM, tiles_n = (p.N + S::kBN - 1) / S::kBN;
+        const int64_t tiles = tiles_m * tiles_n;
+        Params q = p;
+        q.order = stream_order(p.M, p.N, tiles_m, tiles_n);
         if (p.splits > 1) {
-            launch_stream<WM, WN, U, RM, RN, true>(p, dim3(static_cast<uint32_t>(tiles * p.splits)), stream);
+            launch_stream<WM, WN, U, RM, RN, true>(q, dim3(static_cast<uint32_t>(tiles * p.splits)), stream);
         } else {
-            launch_stream<WM, WN, U, RM, RN, false>(p, dim3(static_cast<uint32_t>(tiles)), stream);
+            launch_stream<WM, WN, U, RM, RN, false>(q, dim3(static_cast<uint32_t>(tiles)), stream);
         }
     }
     return true;

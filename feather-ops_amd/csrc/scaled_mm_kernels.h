@@ -377,8 +377,12 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m,
 // The streaming kernel's order. With several rows of tiles, each XCD gets a contiguous run of them, column by column: a
 // column's weight panel is read from memory once, into the L2 of the XCD that holds its rows. Row by row, a panel
 // reaches 8 / gcd(8, columns) L2s: one where the columns are a multiple of 8, where row by row stays (up to 1.2x faster than
-// runs). On 562 shapes and types (M 17-700; weights from HBM) the heuristic's tiles ran 1.16x as fast in geometric mean
-// (0.85-2.1x) with runs off the multiples of 8 as row by row.
+// runs), and two where they are one of 4, where it stays for N < 3 M (358 x 2416 -> 712 bf16 7.4 us against 8.3 in runs;
+// 24 shapes and types 0.91-1.13x, 1.01x in geometric mean; above, the weight's second read counts: runs are 1.02x as fast
+// at N >= 16 M, 1.13x at 28 x 4064 -> 5840). On 562 shapes and types (M 17-700; weights from HBM) the heuristic's tiles ran
+// 1.16x as fast in geometric mean (0.85-2.1x, the lowest at multiples of 4) with runs off the multiples of 8 as row by
+// row. What runs still cost: 0.95-1.02x with columns 2 and 6 past a multiple of 8 at N = 1.3-4 M (893 x 2656 -> 2160 bf16
+// 31.5 against 31.1 us).
 // Tall problems (N < 4/3 M, activations at least 1.5 times the weights) get runs row by row instead: each XCD reads its own
 // rows once and the small weights from its L2, where a run of columns reads all the activations again in every column.
 // On 91 such shapes and types of 7 us and more it is 1.16x faster than column runs in geometric mean (0.98-1.64x, the more
@@ -389,7 +393,7 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m,
 inline TileOrder stream_order(int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n) {
     TileOrder o{};
     const bool tall = 3 * N < 4 * M;
-    const bool runs = tiles_m > 1 && (tall || tiles_n % 8 != 0);
+    const bool runs = tiles_m > 1 && (tall || (tiles_n % 8 != 0 && (tiles_n % 4 != 0 || N >= 3 * M)));
     const bool by_row = !runs || tall;
     o.length = static_cast<uint32_t>(by_row ? tiles_n : tiles_m);
     o.inverse = o.length == 1 ? ~0u : static_cast<uint32_t>((uint64_t{1} << 32) / o.length);

@@ -387,13 +387,17 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m,
 // rows once and the small weights from its L2, where a run of columns reads all the activations again in every column.
 // On 91 such shapes and types of 7 us and more it is 1.16x faster than column runs in geometric mean (0.98-1.64x, the more
 // the fewer columns: 1640 x 2464 -> 736 bf16 18.4 -> 15.1 us, 606 x 7104 -> 232 fp16 15.2 -> 9.2); the gain ends
-// between N = 1.3 M (1.00x) and 1.9 M (0.87x at 891 x 3728 -> 1680).
+// between N = 1.3 M (1.00x) and 1.9 M (0.87x at 891 x 3728 -> 1680). Activations that fit an XCD's 4 MB L2 leave nothing
+// to save, and with an even number of columns, which then go to 8, 4 or 2 XCDs instead of all, id order is faster: 0.97x in
+// geometric mean by runs on 56 such shapes and types (168 x 848 -> 192 bf16 3.1 us against 2.6); with an odd one 1.03x on
+// 49, and past 4 MB 1.19x on 29.
 // The host picks the order and prepares the division: worked out in the kernel ahead of its first load, it cost every block
 // of a call with several rows of tiles 0.1 us (31 x 560 -> 320 2.39 us against 2.27).
-inline TileOrder stream_order(int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n) {
+inline TileOrder stream_order(int64_t M, int64_t N, int64_t K, int64_t tiles_m, int64_t tiles_n) {
     TileOrder o{};
     const bool tall = 3 * N < 4 * M;
-    const bool runs = tiles_m > 1 && (tall || (tiles_n % 8 != 0 && (tiles_n % 4 != 0 || N >= 3 * M)));
+    const bool runs = tiles_m > 1 && (tall ? tiles_n % 2 != 0 || M * K * 2 >= int64_t{4} << 20
+                                           : tiles_n % 8 != 0 && (tiles_n % 4 != 0 || N >= 3 * M));
     const bool by_row = !runs || tall;
     o.length = static_cast<uint32_t>(by_row ? tiles_n : tiles_m);
     o.inverse = o.length == 1 ? ~0u : static_cast<uint32_t>((uint64_t{1} << 32) / o.length);

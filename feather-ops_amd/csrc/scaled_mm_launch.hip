@@ -127,7 +127,7 @@ bool try_tile(const TileQuery& t, const Params& p, hipStream_t stream) {
         const int64_t tiles_m = (p.M + S::kBM - 1) / S::kBM, tiles_n = (p.N + S::kBN - 1) / S::kBN;
         const int64_t tiles = tiles_m * tiles_n;
         Params q = p;
-        q.order = stream_order(p.M, p.N, tiles_m, tiles_n);
+        q.order = stream_order(p.M, p.N, p.K, tiles_m, tiles_n);
         if (p.splits > 1) {
             launch_stream<WM, WN, U, RM, RN, true>(q, dim3(static_cast<uint32_t>(tiles * p.splits)), stream);
         } else {

@@ -65,12 +65,14 @@ struct TileOrder {
     static constexpr uint32_t kByRow = 1u << 31;
 };
 
+// What every block needs before its first load comes first, in the 64 bytes of one scalar load.
+// What the kernels need ahead of their first load fills the first 64 bytes, one scalar load. (With the order among them and
+// c too, split launches of the ring kernel waited for a second one: 33 x 9760 -> 7520 26.4 -> 26.8 us; with the order past
+// them, streaming launches of 2-3 us did, 0.02 us.)
 struct Params {
     const uint16_t* a;          // [M, K] fp16 or bf16 bits, row-major
     const uint8_t* b;           // [kb_total, N, 16] fp8 codes
     const float* scale;         // 1 fp32 value (col_scale == 0) or N (col_scale != 0), or nullptr
-    const uint16_t* bias;       // [N] in the output dtype, or nullptr
-    uint16_t* c;                // [M, N] output bits, row-major
     int32_t M, N, K;
     TileOrder order;            // streaming kernel: set by the launcher
     int32_t kb_total;           // b_prepacked.shape[0]
@@ -78,11 +80,13 @@ struct Params {
     // Split-K (ring kernel only): each output tile's 64-deep stages are cut into `splits` contiguous
     // ranges, one workgroup per range. 1 = no split; then the two pointers are unused.
     int32_t splits;
-    uint32_t* split_ctr;        // [tiles * waves] arrival counters: zero before a launch, zero after it
-    uint8_t* split_part;        // [tiles][splits][waves][RM * RN][64 lanes] fp32x4 partial sums
     // Ring kernel: workgroups [0, reads_first_blocks) take the reads-first operand schedule, the rest the
     // interleaved one (0: all interleaved). The launcher picks it from the grid's CU occupancy.
     int32_t reads_first_blocks;
+    const uint16_t* bias;       // [N] in the output dtype, or nullptr
+    uint16_t* c;                // [M, N] output bits, row-major
+    uint32_t* split_ctr;        // [tiles * waves] arrival counters: zero before a launch, zero after it
+    uint8_t* split_part;        // [tiles][splits][waves][RM * RN][64 lanes] fp32x4 partial sums
     // The weight may be loaded non-temporally (set by the C ABI from the weight's size and the process-wide
     // mode): the launcher does so for tiles whose launch reads each weight byte once (M within one tile row).
     int32_t stream_weight;

@@ -147,25 +147,83 @@ void scaled_mm(const Tensor& a, const Tensor& b_prepacked, const std::optional<T
     check_launch(launched, "scaled_mm");
 }
 
-// feather_ops::scaled_mm_new: scaled_mm into a new output [M, N], fp16 or bf16, with the tile's six numbers packed into one
-// (8 bits each, the first lowest): the auto path's call, where the host's time counts. The allocation here and the shorter
-// argument list save a fifth of a decode-sized call (8.4 -> 6.7 us a call at 1 x 2560 x 1000, whose kernel takes 3.9).
-Tensor scaled_mm_new(const Tensor& a, const Tensor& b_prepacked, const std::optional<Tensor>& scale,
-                     const std::optional<Tensor>& bias, const bool out_bf16, const int64_t tile) {
-    STD_TORCH_CHECK(a.is_cuda(), "a must be a CUDA tensor");
-    STD_TORCH_CHECK(a.dim() == 2, "a must be 2D");
-    STD_TORCH_CHECK(b_prepacked.dim() == 3, "b_prepacked must be 3D (K/16, N, 16)");
-    const int64_t sizes[2] = {a.size(0), b_prepacked.size(1)};
-    const int64_t strides[2] = {sizes[1], 1};
+// An uninitialized contiguous [rows, cols] tensor of one of the 16-bit types on a's device.
+Tensor new_matrix(const Tensor& a, const int64_t rows, const int64_t cols, const bool bf16) {
+    const int64_t sizes[2] = {rows, cols};
+    const int64_t strides[2] = {cols, 1};
     int32_t device_type = 0;
     TORCH_ERROR_CODE_CHECK(aoti_torch_get_device_type(a.get(), &device_type));
     AtenTensorHandle handle = nullptr;
     TORCH_ERROR_CODE_CHECK(aoti_torch_empty_strided(2, sizes, strides,
-                                                    out_bf16 ? aoti_torch_dtype_bfloat16() : aoti_torch_dtype_float16(),
+                                                    bf16 ? aoti_torch_dtype_bfloat16() : aoti_torch_dtype_float16(),
                                                     device_type, a.get_device_index(), &handle));
-    Tensor c(handle);
-    const auto field = [tile](int i) { return (tile >> (8 * i)) & 0xff; };
-    scaled_mm(a, b_prepacked, scale, bias, c, field(0), field(1), field(2), field(3), field(4), field(5) != 0);
+    return Tensor(handle);
+}
+
+Tensor new_output(const Tensor& a, const Tensor& b_prepacked, const bool out_bf16) {
+    STD_TORCH_CHECK(a.is_cuda(), "a must be a CUDA tensor");
+    STD_TORCH_CHECK(a.dim() == 2, "a must be 2D");
+    STD_TORCH_CHECK(b_prepacked.dim() == 3, "b_prepacked must be 3D (K/16, N, 16)");
+    return new_matrix(a, a.size(0), b_prepacked.size(1), out_bf16);
+}
+
+// Number i of a tile's six, packed into one (8 bits each, the first lowest).
+int tile_field(const int64_t tile, const int i) { return static_cast<int>((tile >> (8 * i)) & 0xff); }
+
+// feather_ops::scaled_mm_new: scaled_mm into a new output [M, N], fp16 or bf16, with the tile's six numbers packed into
+// one: the auto path's call, where the host's time counts. The allocation here and the shorter
+// argument list save a fifth of a decode-sized call (8.4 -> 6.7 us a call at 1 x 2560 x 1000, whose kernel takes 3.9).
+Tensor scaled_mm_new(const Tensor& a, const Tensor& b_prepacked, const std::optional<Tensor>& scale,
+                     const std::optional<Tensor>& bias, const bool out_bf16, const int64_t tile) {
+    Tensor c = new_output(a, b_prepacked, out_bf16);
+    scaled_mm(a, b_prepacked, scale, bias, c, tile_field(tile, 0), tile_field(tile, 1), tile_field(tile, 2),
+              tile_field(tile, 3), tile_field(tile, 4), tile_field(tile, 5) != 0);
+    return c;
+}
+
+// feather_ops::scaled_mm_parts_new: the same in two launches, the first `rows` rows on one tile and the rest on another
+// with `splits` K ranges (workspace: as scaled_mm_splitk's, for that launch), `widen`: after bf16 activations are widened
+// to fp16. One op, because the GPU waits for the host between the launches of a call that finds it idle: separate ops
+// took 24 us of host time at 4097 x 2560 -> 5120 in bf16, 13 here (one launch: 8), and a call on its own 112 us, 109 here.
+Tensor scaled_mm_parts_new(const Tensor& a, const Tensor& b_prepacked, const std::optional<Tensor>& scale,
+                           const std::optional<Tensor>& bias, const bool out_bf16, const bool widen, const int64_t rows,
+                           const int64_t tile, const int64_t last_tile, const int64_t splits,
+                           std::optional<Tensor> workspace) {
+    Tensor c = new_output(a, b_prepacked, out_bf16);
+    const Operands o =
+        check_operands(a, b_prepacked, scale, bias, c, tile_field(tile, 0), tile_field(tile, 1));
+    STD_TORCH_CHECK(rows > 0 && rows < o.M && rows % 8 == 0, "rows must be a multiple of 8 between 0 and M");
+    STD_TORCH_CHECK(splits == 1 || (workspace.has_value() && workspace->is_cuda() &&
+                                    workspace->get_device_index() == o.device_index &&
+                                    workspace->scalar_type() == ST::Byte && workspace->is_contiguous()),
+                    "splits need a contiguous uint8 workspace on the same device as a");
+    torch::stable::accelerator::DeviceGuard guard(o.device_index);
+    const hipStream_t stream = current_stream(o.device_index);
+    const auto* x = static_cast<const uint16_t*>(a.const_data_ptr());
+    std::optional<Tensor> wide;   // back to the allocator at the end, for later work of this stream
+    if (widen && o.a_bf16) {
+        wide = new_matrix(a, o.M, o.K, false);
+        auto* const out = static_cast<uint16_t*>(wide->mutable_data_ptr());
+        check_launch(feather_widen_bf16(x, out, o.M * o.K, stream), "widen_bf16");
+        x = out;
+    }
+    const auto* const b = static_cast<const uint8_t*>(b_prepacked.const_data_ptr());
+    const auto* const s = scale.has_value() ? static_cast<const float*>(scale->const_data_ptr()) : nullptr;
+    const auto* const add = bias.has_value() ? static_cast<const uint16_t*>(bias->const_data_ptr()) : nullptr;
+    auto* const y = static_cast<uint16_t*>(c.mutable_data_ptr());
+    const bool a_bf16 = o.a_bf16 && !widen;
+    check_launch(launch_scaled_mm(x, b, s, add, y, rows, o.N, o.K, o.scale_mode, add != nullptr, o.e5m2, a_bf16, o.out_bf16,
+                                  tile_field(tile, 0), tile_field(tile, 1), tile_field(tile, 2), tile_field(tile, 3),
+                                  tile_field(tile, 4), tile_field(tile, 5) != 0, stream),
+                 "scaled_mm");
+    check_launch(feather_scaled_mm_splitk(x + rows * o.K, b, s, add, y + rows * o.N, o.M - rows, o.N, o.K, o.scale_mode,
+                                          add != nullptr, o.e5m2, a_bf16, o.out_bf16, tile_field(last_tile, 0),
+                                          tile_field(last_tile, 1), tile_field(last_tile, 2), tile_field(last_tile, 3),
+                                          tile_field(last_tile, 4), tile_field(last_tile, 5) != 0,
+                                          static_cast<int>(splits),
+                                          workspace.has_value() ? workspace->mutable_data_ptr() : nullptr,
+                                          workspace.has_value() ? workspace->numel() : 0, stream),
+                 "scaled_mm");
     return c;
 }
 
@@ -385,6 +443,9 @@ STABLE_TORCH_LIBRARY(feather_ops, m) {
         "int repeat_n, bool prefetch=True) -> ()");
     m.def(
         "scaled_mm_new(Tensor a, Tensor b_prepacked, Tensor? scale, Tensor? bias, bool out_bf16, int tile) -> Tensor");
+    m.def(
+        "scaled_mm_parts_new(Tensor a, Tensor b_prepacked, Tensor? scale, Tensor? bias, bool out_bf16, bool widen, int rows, "
+        "int tile, int last_tile, int splits, Tensor(a!)? workspace) -> Tensor");
     m.def("bf16_to_fp16(Tensor x, Tensor(a!) out) -> ()");
     m.def("widen_bf16(Tensor x, Tensor(a!) out) -> ()");
     m.def("prepack_b(Tensor b, Tensor(a!) out) -> ()");
@@ -400,6 +461,7 @@ STABLE_TORCH_LIBRARY_IMPL(feather_ops, CUDA, m) {
     m.impl("scaled_mm", TORCH_BOX(&scaled_mm));
     m.impl("scaled_mm_splitk", TORCH_BOX(&scaled_mm_splitk));
     m.impl("scaled_mm_new", TORCH_BOX(&scaled_mm_new));
+    m.impl("scaled_mm_parts_new", TORCH_BOX(&scaled_mm_parts_new));
     m.impl("bf16_to_fp16", TORCH_BOX(&bf16_to_fp16));
     m.impl("widen_bf16", TORCH_BOX(&widen_bf16));
     m.impl("prepack_b", TORCH_BOX(&prepack_b));

@@ -765,13 +765,18 @@ def _auto_parts(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple[tuple[tup
 
 
 @functools.lru_cache(maxsize=4096)
-def _auto_plan(M: int, N: int, K: int,
-               a_dtype: torch.dtype) -> tuple[tuple[tuple[int, tuple[int, ...], int], ...], bool, int | None]:
-    """`_auto_parts` and, where that is one plain launch (unsplit, activations as given), its tile's six numbers packed into
-    one for `feather_ops::scaled_mm_new` (else None): one lookup per call."""
+def _auto_plan(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple:
+    """(`_auto_parts`' launches, widen first, one op's arguments): one lookup per call. The last are, where one plain launch
+    (unsplit, activations as given) is all there is, its tile's six numbers packed into one for
+    `feather_ops::scaled_mm_new`; where the last rows are apart, `feather_ops::scaled_mm_parts_new`'s (widen, rows, tile, last
+    tile, splits) and the workspace bytes; else None."""
     parts, widen = _auto_parts(M, N, K, a_dtype)
-    plain = len(parts) == 1 and not widen and parts[0][2] == 1
-    return parts, widen, sum(field << 8 * i for i, field in enumerate(parts[0][1])) if plain else None
+    tiles = [sum(field << 8 * i for i, field in enumerate(tile)) for _, tile, _ in parts]
+    if len(parts) == 2:
+        (rows, _, first_splits), (last, tile, splits) = parts
+        nbytes = _workspace_bytes(last, N, K, tile, splits) if splits > 1 else 0
+        return parts, widen, (widen, rows, *tiles, splits, nbytes) if first_splits == 1 and nbytes >= 0 else None
+    return parts, widen, tiles[0] if not widen and parts[0][2] == 1 else None
 
 
 # Split-K workspaces, one per (device, stream): the counter area at their start must be zero before a
@@ -800,6 +805,12 @@ def _split_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _split_workspaces[key] = ws
     return ws
+
+
+def _workspace_for(a: torch.Tensor, nbytes: int) -> torch.Tensor:
+    if isinstance(a, FakeTensor):  # made in the traced program, not in the cache that real calls read
+        return torch.zeros(nbytes, dtype=torch.uint8, device=a.device)
+    return _split_workspace(a.device, nbytes)
 
 
 def clear_split_workspaces() -> None:
@@ -863,10 +874,7 @@ def _launch(
         if nbytes < 0:
             raise RuntimeError(
                 f"split-K needs an instantiated tile and 1 <= splits <= the K units, got {tile}, {splits}")
-        if isinstance(a, FakeTensor):  # made in the traced program, not in the cache that real calls read
-            ws = torch.zeros(nbytes, dtype=torch.uint8, device=a.device)
-        else:
-            ws = _split_workspace(a.device, nbytes)
+        ws = _workspace_for(a, nbytes)
     torch.ops.feather_ops.scaled_mm_splitk.default(a, b_prepacked, scale, bias, out, ws, splits, *tile)
 
 
@@ -899,11 +907,11 @@ def _launch_auto(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor
 
 _lib.load()
 _scaled_mm_new = torch.ops.feather_ops.scaled_mm_new.default
+_scaled_mm_parts_new = torch.ops.feather_ops.scaled_mm_parts_new.default
 
 
-@torch.library.register_fake("feather_ops::scaled_mm_new")
-def _(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bias: torch.Tensor | None, out_bf16: bool,
-      tile: int) -> torch.Tensor:
+def _fake_output(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bias: torch.Tensor | None,
+                 out_bf16: bool, *plan) -> torch.Tensor:
     # Fake tensors only (shape propagation, make_fx): like the ops that write into an output, none of them for the
     # meta device itself.
     if a.device.type == "meta":
@@ -911,10 +919,14 @@ def _(a: torch.Tensor, b_prepacked: torch.Tensor, scale: torch.Tensor | None, bi
     return a.new_empty((a.shape[0], b_prepacked.shape[1]), dtype=torch.bfloat16 if out_bf16 else torch.float16)
 
 
-@torch.library.register_vmap("feather_ops::scaled_mm_new")
-def _(info, in_dims, *args):
-    # as the ops that write into an output do; vmap's loop would take some shapes (one plain launch) and refuse others
+def _no_batching(info, in_dims, *args):
+    # as the ops that write into an output do; vmap's loop would take some shapes and refuse others
     raise RuntimeError("Batching rule not implemented for feather_ops::scaled_mm_new")
+
+
+for _op in ("feather_ops::scaled_mm_new", "feather_ops::scaled_mm_parts_new"):
+    torch.library.register_fake(_op, _fake_output)
+    torch.library.register_vmap(_op, _no_batching)
 
 
 @custom_op("feather_ops::scaled_mm_auto", mutates_args=("out",))
@@ -948,20 +960,24 @@ def scaled_mm_hip(
     The heuristic's launch goes through the opaque custom op `feather_ops::scaled_mm_auto` while
     `torch.compile` traces (as in the reference, `scaled_mm.py:104-134`), and straight to the launcher in
     eager mode: the same launch without the custom op's Python dispatch, about 7 us of host time per call,
-    which is more than a decode-sized kernel takes. Where that is one plain launch, one op allocates the output
-    and launches it.
+    which is more than a decode-sized kernel takes. Where that is one plain launch, or two with the last rows
+    apart, one op allocates the output and launches it.
     """
     _lib.require_native()
     auto = tile is None and splits is None
     plan = None
     if auto and not torch.compiler.is_compiling():
         shape = a.shape
-        *plan, packed = _auto_plan(shape[0], b_prepacked.shape[1], shape[1], a.dtype)
+        *plan, one_op = _auto_plan(shape[0], b_prepacked.shape[1], shape[1], a.dtype)
         # operands that autograd follows take the ops that write into an output: it marks what an op returns
-        if packed is not None and (out_dtype is torch.bfloat16 or out_dtype is torch.float16) and not (
+        if one_op is not None and (out_dtype is torch.bfloat16 or out_dtype is torch.float16) and not (
                 a.requires_grad or b_prepacked.requires_grad or (scale is not None and scale.requires_grad)
                 or (bias is not None and bias.requires_grad)):
-            return _scaled_mm_new(a, b_prepacked, scale, bias, out_dtype is torch.bfloat16, packed)
+            if type(one_op) is int:
+                return _scaled_mm_new(a, b_prepacked, scale, bias, out_dtype is torch.bfloat16, one_op)
+            *one_op, nbytes = one_op
+            return _scaled_mm_parts_new(a, b_prepacked, scale, bias, out_dtype is torch.bfloat16, *one_op,
+                                        _workspace_for(a, nbytes) if nbytes else None)
     out = torch.empty((a.shape[0], b_prepacked.shape[1]), device=a.device, dtype=out_dtype)
     if plan is not None:
         _launch_auto(a, b_prepacked, scale, bias, out, plan)

@@ -23,9 +23,9 @@ def test_shapes_cover_the_launches():
     kinds = set()
     for m, n, k in SHAPES:
         for dtype in (FP16, BF16):
-            parts, widen, packed = impl._auto_plan(m, n, k, dtype)
-            kinds |= {"plain" if packed is not None else "widened" if widen else "split" if len(parts) == 1 else "parts"}
-            kinds |= {"parts"} if len(parts) > 1 else set()
+            parts, widen, one_op = impl._auto_plan(m, n, k, dtype)
+            kinds.add("parts" if len(parts) > 1 else "widened" if widen else "split" if parts[0][2] > 1 else "plain")
+            assert (one_op is None) == (len(parts) == 1 and (widen or parts[0][2] > 1))
     assert kinds == {"plain", "split", "widened", "parts"}
 
 
@@ -52,10 +52,11 @@ def test_make_fx(m, n, k, mode):
     nodes = [node for node in graph.nodes if node.op != "placeholder"]
     assert not any(node.op == "get_attr" for node in nodes)
     for node in nodes:
-        if node.target is torch.ops.feather_ops.scaled_mm_splitk.default:
-            assert node.args[5].target is torch.ops.aten.zeros.default   # its counters start at zero
-    launches = [node for node in nodes if "feather_ops" in str(node.target)]
-    assert len(launches) == len(impl._auto_plan(m, n, k, FP16)[0])
+        splits = {torch.ops.feather_ops.scaled_mm_splitk.default: (6, 5),
+                  torch.ops.feather_ops.scaled_mm_parts_new.default: (9, 10)}.get(node.target)
+        if splits is not None and node.args[splits[0]] > 1:
+            assert node.args[splits[1]].target is torch.ops.aten.zeros.default   # its counters start at zero
+    assert sum("feather_ops" in str(node.target) for node in nodes) == 1
 
 
 def test_relabelled_linear_without_gradients():

@@ -5,7 +5,7 @@ import random
 import pytest
 import torch
 
-from feather_ops.scaled_mm import _TAIL_MAX_ROWS, _auto_choice, _auto_parts, _refined
+from feather_ops.scaled_mm import _TAIL_MAX_ROWS, _auto_choice, _auto_parts, _launch_auto, _refined
 
 FP16, BF16 = torch.float16, torch.bfloat16
 
@@ -76,6 +76,40 @@ def test_outputs(m, n, k, dtype):
         out = feather_ops.scaled_mm_hip(a, b, scale, bias, dtype)
         rows = sorted({0, 1, 255, 256, m // 2, *range(m - m % 128 - 2, m)})
         check_against_oracle(out, a, b, scale, bias, rows=rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("m,n,k", SPLIT)
+def test_one_op_and_the_launches_one_by_one_agree(m, n, k, dtype):
+    """scaled_mm_parts_new against the ops that write into an output, which calls that autograd follows still take."""
+    import feather_ops
+
+    a, b, scale, bias = _inputs(m, n, k, dtype, True)
+    for out_dtype in (FP16, BF16):
+        add = bias.to(out_dtype)
+        for s in (None, scale[0], scale):
+            got = feather_ops.scaled_mm_hip(a, b, s, add, out_dtype)
+            want = torch.empty_like(got)
+            _launch_auto(a, b, s, add, want)
+            assert got.is_contiguous() and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_other_streams():
+    import feather_ops
+
+    a, b, scale, bias = _inputs(*SPLIT[5], BF16, True)
+    want = feather_ops.scaled_mm_hip(a, b, scale, bias, BF16)
+    outs = []
+    for _ in range(3):
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            outs.append(feather_ops.scaled_mm_hip(a, b, scale, bias, BF16))
+        torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, want) for out in outs)
 
 
 @pytest.mark.gpu

@@ -808,7 +808,8 @@ def _split_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 
 
 def _workspace_for(a: torch.Tensor, nbytes: int) -> torch.Tensor:
-    if isinstance(a, FakeTensor):  # made in the traced program, not in the cache that real calls read
+    # Of fake tensors (made in the traced program) and off the GPU (the op refuses it): not for the cache of a stream.
+    if isinstance(a, FakeTensor) or not a.is_cuda:
         return torch.zeros(nbytes, dtype=torch.uint8, device=a.device)
     return _split_workspace(a.device, nbytes)
 

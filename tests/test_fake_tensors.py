@@ -69,8 +69,11 @@ def test_relabelled_linear_without_gradients():
 def test_what_the_two_step_call_refuses():
     with pytest.raises(NotImplementedError, match="Meta"):
         feather_ops.scaled_mm_hip(*_operands(16, 1000, 2560, FP16, "meta"), None, FP16)
-    with pytest.raises(NotImplementedError, match="CPU"):
-        feather_ops.scaled_mm_hip(*_operands(16, 1000, 2560, FP16, "cpu"), None, FP16)
+    before = dict(impl._split_workspaces)
+    for m, n, k in SHAPES[:4] + SHAPES[5:]:
+        with pytest.raises(NotImplementedError, match="CPU"):
+            feather_ops.scaled_mm_hip(*_operands(m, n, k, FP16, "cpu"), None, FP16)
+    assert impl._split_workspaces == before
     with FakeTensorMode():
         _, b, scale = _operands(16, 1000, 2560, FP16)
         with pytest.raises(RuntimeError, match="Batching rule not implemented"):

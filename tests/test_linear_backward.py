@@ -67,6 +67,25 @@ def test_operands_off_the_gpu_take_torch(column):
     assert none_x.numel() == none_b.numel() == 0
 
 
+def test_what_the_kernels_do_not_take_stays_out_of_the_op(monkeypatch):
+    """A small layer's backward is torch's operations without the op's Python dispatch, rounded once."""
+    import types
+
+    from feather_ops.modules import _linear_backward
+
+    def op(*args):
+        raise AssertionError("the op")
+
+    monkeypatch.setattr(lb, "linear_backward", op)
+    torch.manual_seed(0)
+    wq, scale, grad = torch.randn(24, 48).to(torch.float8_e5m2), torch.rand(24), torch.randn(10, 24).to(torch.bfloat16)
+    ctx = types.SimpleNamespace(saved_tensors=(prepack_transpose(wq), scale), x_shape=(10, 48), x_dtype=torch.float16,
+                                bias_dtype=torch.float32, needs_input_grad=(True, False, False, True))
+    gx, _, _, gb = _linear_backward(ctx, grad)
+    assert torch.equal(gx, (grad.float() @ (wq.float() * scale[:, None])).to(torch.float16))
+    assert torch.equal(gb, grad.float().sum(0))
+
+
 def test_tangents_of_gradients():
     """Forward mode over the backward (a Hessian-vector product): the gradient's tangent reaches both results."""
     import types

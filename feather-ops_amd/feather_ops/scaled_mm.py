@@ -999,8 +999,8 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
     `K` is zero-padded to a multiple of 128, so a ragged K never needs a staging branch; element
     `[k // 16, n, k % 16]` of the result is `b[k, n]`. A contiguous e5m2 / e4m3fn weight on the GPU with
     N a multiple of 8 is permuted by one HIP kernel (`csrc/prepack.hip`, HBM-bound), and so is the transposed
-    view of a contiguous `[N, K]` one with K a multiple of 16; anything else (a CPU weight, another dtype or
-    width) by torch copy kernels on `b`'s device. Run once per weight.
+    view of a contiguous `[N, K]` one with K a multiple of 16 and over 2 MiB; anything else (a CPU weight, another dtype
+    or width) by torch copy kernels on `b`'s device. Run once per weight.
     """
     k, n = b.shape
     k_pad = -(-k // 128) * 128
@@ -1009,7 +1009,7 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
         out = torch.empty((k_pad // 16, n, 16), device=b.device, dtype=b.dtype)
         torch.ops.feather_ops.prepack_b.default(b, out)
         return out
-    if b.dtype in _FP8_DTYPES and b.stride(0) == 1:
+    if b.dtype in _FP8_DTYPES and b.stride(0) == 1 and not _small_rows(n, k):
         w = b.t()
         if _packs_rows(w):
             return _pack_rows(w)
@@ -1018,6 +1018,12 @@ def prepack_b_for_scaled_mm(b: torch.Tensor) -> torch.Tensor:
         padded[:k] = b
         b = padded
     return b.view(k_pad // 16, 16, n).permute(0, 2, 1).contiguous()
+
+
+def _small_rows(n: int, k: int) -> bool:
+    """Whether a [N, K] fp8 weight is small enough for torch's one copy, bound by the host there: 7.2 us a call against 8.3 by
+    the kernel up to 2 MiB (8.4 and 8.3 at 4 MiB, 14.2 and 8.3 at 8). Without padding only, which takes torch three."""
+    return k % 128 == 0 and n * k <= 1 << 21
 
 
 def _packs_rows(w: torch.Tensor) -> bool:
@@ -1065,11 +1071,11 @@ def prepack_transpose(w: torch.Tensor) -> torch.Tensor:
 
     For a row of `w` the 16 k values of a chunk are already 16 contiguous bytes, so the prepack is a
     transpose of `[N, K_pad/16]` 16-byte units: one HIP kernel (`csrc/prepack.hip`) where it takes the weight
-    (`_packs_rows`), torch copies otherwise.
+    (`_packs_rows`) and the weight is over 2 MiB or padded, torch copies otherwise.
     """
     n, k = w.shape
     k_pad = -(-k // 128) * 128
-    if w.dtype in _FP8_DTYPES and _packs_rows(w):
+    if w.dtype in _FP8_DTYPES and not _small_rows(n, k) and _packs_rows(w):
         return _pack_rows(w)
     if k_pad != k:
         padded = torch.zeros((n, k_pad), device=w.device, dtype=w.dtype)

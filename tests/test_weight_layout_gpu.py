@@ -40,8 +40,9 @@ def _check_quantized(w, fp8, per_channel):
     assert torch.equal(codes.view(torch.uint8), _packed(want))
 
 
-# (n, k): one unit; a tail of rows, of units, of both; whole tiles; a K with no pad
-SHAPES = [(1, 16), (33, 48), (264, 640), (1000, 2560), (32, 512), (40, 1040), (4096, 128)]
+# (n, k): one unit; a tail of rows, of units, of both; whole tiles; a K with no pad; the sides of 2 MiB, where codes without
+# a pad go from torch's copy to the kernel
+SHAPES = [(1, 16), (33, 48), (264, 640), (1000, 2560), (32, 512), (40, 1040), (4096, 128), (4096, 512), (4104, 512)]
 
 
 @pytest.mark.parametrize("n,k", SHAPES)

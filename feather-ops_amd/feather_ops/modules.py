@@ -125,21 +125,23 @@ def _linear_setup_context(ctx, inputs, output) -> None:
 def _linear_backward(ctx, grad: torch.Tensor):
     """Gradients for the activations and the bias (the fp8 weight is frozen): dX = dY @ (Wq * scale)^T as fp32
     arithmetic gives it on the dequantized weight, dbias = the column sums of dY."""
-    from .linear_backward import composite, linear_backward, takes
+    from . import linear_backward as lb
 
     weight_fp8, weight_scale = ctx.saved_tensors
     k = ctx.x_shape[-1]
-    need_x, need_bias = ctx.needs_input_grad[0], ctx.bias_dtype is not None and ctx.needs_input_grad[3]
+    need_x, _, _, need_bias = ctx.needs_input_grad
+    plain = type(grad) is torch.Tensor
     # A gradient that is itself differentiated (create_graph, or a tangent of forward mode) or batched by a transform
     # (vmap, grad of grad) takes torch's operations, which have rules for all of them; so does one that the kernels do not
     # take, here and not inside the op, whose Python dispatch costs a small layer 45 us a pass. A traced gradient (a
     # subclass) is left to the op.
-    if ((torch.is_grad_enabled() and grad.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(grad)
+    if ((plain and grad.numel() * k < lb._MIN_PRODUCTS) or (torch.is_grad_enabled() and grad.requires_grad)
+            or torch._C._functorch.is_functorch_wrapped_tensor(grad)
             or forward_ad.unpack_dual(grad).tangent is not None
-            or (type(grad) is torch.Tensor and not takes(grad, weight_fp8, weight_scale, k))):
-        grad_x, grad_bias = composite(grad, weight_fp8, weight_scale, k)
+            or (plain and not lb.takes(grad, weight_fp8, weight_scale, k))):
+        grad_x, grad_bias = lb.composite(grad, weight_fp8, weight_scale, k)
     else:
-        grad_x, grad_bias = linear_backward(grad, weight_fp8, weight_scale, k, need_x, need_bias)
+        grad_x, grad_bias = lb.linear_backward(grad, weight_fp8, weight_scale, k, need_x, need_bias)
     return (grad_x.to(ctx.x_dtype).reshape(ctx.x_shape) if need_x else None, None, None,
             grad_bias.to(ctx.bias_dtype) if need_bias else None)
 

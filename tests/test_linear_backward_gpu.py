@@ -128,6 +128,32 @@ def test_infinities_and_nan(lb, every_size, fp8, column):
         assert torch.equal(got[got.isinf()], want[want.isinf()])
 
 
+@pytest.mark.parametrize("fp8", [E5M2, E4M3])
+@pytest.mark.parametrize("dtype,power", [(FP16, 12), (BF16, 12), (BF16, -20)])
+@pytest.mark.parametrize("m,n,k", [(70, 264, 272), (300, 1000, 1008), (1000, 1024, 512), (1040, 6144, 1536)])
+def test_results_of_the_last_term_alone(lb, every_size, m, n, k, dtype, power, fp8):
+    """Columns in pairs of opposite gradients and equal codes, whose scales differ in the 8 lowest bits: the first two of the
+    gradient's three terms cancel. Gradients are +-1, codes of 3 significant bits and scales of one binade, so every sum
+    is exact in fp32 (the first term's in steps of 2^-9 under 2^15, the last's of 2^-25) and only the result is rounded."""
+    from feather_ops import prepack_transpose
+
+    g = torch.Generator("cuda").manual_seed(0)
+    sign = torch.randint(0, 2, (m, n // 2), generator=g, device="cuda") * 2 - 1
+    grad = torch.stack([sign, -sign], 2).view(m, n).to(dtype)
+    codes = torch.randint(4, 8, (n // 2, k), generator=g, device="cuda") * 0.25
+    codes = codes * (torch.randint(0, 2, codes.shape, generator=g, device="cuda") * 2 - 1)
+    wq = codes.repeat_interleave(2, 0).to(fp8)
+    assert torch.equal(wq.float(), codes.repeat_interleave(2, 0))
+    bits = torch.randint(0, 1 << 15, (n // 2,), generator=g, device="cuda").repeat_interleave(2) << 8
+    low = torch.randint(0, 1 << 8, (n,), generator=g, device="cuda")
+    scale, without = (((bits + x).double() * 2.0**-23 + 1.0) * 2.0**power for x in (low, torch.zeros_like(low)))
+    x, _ = lb.linear_backward(grad, prepack_transpose(wq), scale.float(), k, True, False)
+    want, two_terms = ((grad.double() * s) @ wq.double() for s in (scale, without))
+    half, least = (2.0**-8, 2.0**-134) if dtype == BF16 else (2.0**-11, 2.0**-25)
+    assert two_terms.abs().max() == 0.0 and want.abs().max() > 2.0**(power - 14)
+    assert ((x.double() - want).abs() <= half * want.abs() + least).all()
+
+
 def _layer(dtype=BF16, k=1024, n=4104, column=True):
     import feather_ops
 

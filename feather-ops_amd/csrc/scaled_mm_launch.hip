@@ -29,11 +29,10 @@ constexpr int kCus = 256;                // MI355X compute units
 template <int WM, int WN, int U, int RM, int RN, bool kSplitK, bool kDeep>
 void launch_ring(const Params& q, dim3 grid, hipStream_t stream) {
     using S = DmaShape<WM, WN, U, RM, RN>;
-    if constexpr (S::kBM <= 64) {
+    if constexpr (S::kBM <= 64 && !kBf16Mfma) {   // the gradient matmul's weight comes from the caches
         if (q.stream_weight && q.M <= S::kBM) {
-            hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep, true,
-                                                kBf16Mfma>),
-                               grid, dim3(S::kThreads), 0, stream, q);
+            hipLaunchKernelGGL((ring_dma_kernel<WM, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, kDeep, true>), grid,
+                               dim3(S::kThreads), 0, stream, q);
             return;
         }
     }
@@ -44,13 +43,15 @@ void launch_ring(const Params& q, dim3 grid, hipStream_t stream) {
 template <int KS, int WN, int U, int RM, int RN, bool kSplitK>
 void launch_stream(const Params& p, dim3 grid, hipStream_t stream) {
     using S = StreamShape<KS, WN, U, RM, RN>;
-    if (p.stream_weight && p.M <= S::kBM) {
-        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, true, kBf16Mfma>),
-                           grid, dim3(S::kThreads), 0, stream, p);
-    } else {
-        hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, false, kBf16Mfma>),
-                           grid, dim3(S::kThreads), 0, stream, p);
+    if constexpr (!kBf16Mfma) {
+        if (p.stream_weight && p.M <= S::kBM) {
+            hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, true>), grid,
+                               dim3(S::kThreads), 0, stream, p);
+            return;
+        }
     }
+    hipLaunchKernelGGL((stream_kernel<KS, WN, U, RM, RN, kE5M2, kABf16, kOutBf16, kSplitK, false, kBf16Mfma>), grid,
+                       dim3(S::kThreads), 0, stream, p);
 }
 
 template <int WM, int WN, int U, int RM, int RN, int PF>

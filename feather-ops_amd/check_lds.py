@@ -11,6 +11,7 @@ combination to assembly (device code only, ~10 s) and reads `.amdhsa_group_segme
 
     python check_lds.py                 # e5m2 weights, fp16 activations, fp16 output
     python check_lds.py --combo 011     # <e5m2><a_bf16><out_bf16>
+    python check_lds.py --combo 021     # a_bf16 = 2: the gradient matmul's, on GRAD_TILES
 """
 
 import argparse
@@ -23,6 +24,7 @@ import sys
 HERE = pathlib.Path(__file__).resolve().parent
 ROOT = HERE.parent
 HIPCC = "/opt/rocm/bin/hipcc"
+COMBOS = [f"{e5m2}{a}{out}" for e5m2 in (0, 1) for a in (0, 1, 2) for out in (0, 1)]
 
 
 def _tiles():
@@ -101,8 +103,8 @@ def audit(asm: str) -> tuple[int, list[tuple]]:
 
 def main() -> int:
     parser = argparse.ArgumentParser()
-    parser.add_argument("--combo", default="100", choices=[f"{i:03b}" for i in range(8)],
-                        help="<e5m2><a_bf16><out_bf16>")
+    parser.add_argument("--combo", default="100", choices=COMBOS,
+                        help="<e5m2><a_bf16><out_bf16>; a_bf16 = 2: the gradient matmul's")
     args = parser.parse_args()
     checked, bad = audit(compile_asm(args.combo))
     print(f"{checked} kernel instantiations checked against their tile's LDS size")

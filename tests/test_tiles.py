@@ -2,6 +2,7 @@
 duplicates, every tile fits gfx950's limits, and every compiled kernel allocates exactly its tile's LDS."""
 
 import pathlib
+import re
 import subprocess
 import sys
 
@@ -131,3 +132,19 @@ def test_every_kernel_allocates_exactly_its_tiles_lds():
         assert len(check.audit(asm)[1]) == checked
     finally:
         check.expected_bytes = real
+
+
+def test_the_gradient_kernels_allocate_exactly_their_tiles_lds():
+    """The same for the gradient matmul's instantiations, which have no non-temporal variants."""
+    from feather_ops.tiles import GRAD_TILES
+
+    check = _check_lds()
+    if not pathlib.Path(check.HIPCC).exists():
+        pytest.skip("needs hipcc")
+    assert set(check.COMBOS) == set(re.search(r"COMBOS := ([\d ]+)", (pathlib.Path(check.HERE) / "Makefile").read_text())[1].split())
+    checked, bad = check.audit(check.compile_asm("121"))
+    small_ring = sum(1 for t in GRAD_TILES if t[5] == 1 and 16 * t[0] * t[3] <= 64)
+    wide = sum(1 for t in GRAD_TILES if t in ((2, 2, 4, 8, 8, 1), (2, 2, 4, 8, 6, 1)))
+    assert small_ring and wide == 2
+    assert checked == 2 * len(GRAD_TILES) + 2 * small_ring + 2 * wide
+    assert bad == []

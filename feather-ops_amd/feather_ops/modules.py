@@ -130,15 +130,13 @@ def _linear_backward(ctx, grad: torch.Tensor):
     weight_fp8, weight_scale = ctx.saved_tensors
     k = ctx.x_shape[-1]
     need_x, _, _, need_bias = ctx.needs_input_grad
-    plain = type(grad) is torch.Tensor
     # A gradient that is itself differentiated (create_graph, or a tangent of forward mode) or batched by a transform
-    # (vmap, grad of grad) takes torch's operations, which have rules for all of them; so does one that the kernels do not
-    # take, here and not inside the op, whose Python dispatch costs a small layer 45 us a pass. A traced gradient (a
-    # subclass) is left to the op.
-    if ((plain and grad.numel() * k < lb._MIN_PRODUCTS) or (torch.is_grad_enabled() and grad.requires_grad)
+    # (vmap, grad of grad) takes torch's operations, which have rules for all of them; so does a small layer's, here and not
+    # inside the op, whose Python dispatch costs 45 us a pass. A traced gradient (a subclass) is left to the op.
+    if ((type(grad) is torch.Tensor and grad.numel() * k < lb._MIN_PRODUCTS)
+            or (torch.is_grad_enabled() and grad.requires_grad)
             or torch._C._functorch.is_functorch_wrapped_tensor(grad)
-            or forward_ad.unpack_dual(grad).tangent is not None
-            or (plain and not lb.takes(grad, weight_fp8, weight_scale, k))):
+            or forward_ad.unpack_dual(grad).tangent is not None):
         grad_x, grad_bias = lb.composite(grad, weight_fp8, weight_scale, k)
     else:
         grad_x, grad_bias = lb.linear_backward(grad, weight_fp8, weight_scale, k, need_x, need_bias)

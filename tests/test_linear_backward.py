@@ -67,7 +67,7 @@ def test_operands_off_the_gpu_take_torch(column):
     assert none_x.numel() == none_b.numel() == 0
 
 
-def test_what_the_kernels_do_not_take_stays_out_of_the_op(monkeypatch):
+def test_small_layers_stay_out_of_the_op(monkeypatch):
     """A small layer's backward is torch's operations without the op's Python dispatch, rounded once."""
     import types
 

@@ -770,6 +770,8 @@ def _auto_plan(M: int, N: int, K: int, a_dtype: torch.dtype) -> tuple:
     (unsplit, activations as given) is all there is, its tile's six numbers packed into one for
     `feather_ops::scaled_mm_new`; where the last rows are apart, `feather_ops::scaled_mm_parts_new`'s (widen, rows, tile, last
     tile, splits) and the workspace bytes; else None."""
+    # torch.jit.trace passes sizes as tensors
+    M, N, K = (int(size) if isinstance(size, torch.Tensor) else size for size in (M, N, K))
     parts, widen = _auto_parts(M, N, K, a_dtype)
     tiles = [sum(field << 8 * i for i, field in enumerate(tile)) for _, tile, _ in parts]
     if len(parts) == 2:

@@ -5,7 +5,7 @@ import random
 import pytest
 import torch
 
-from feather_ops.scaled_mm import _TAIL_MAX_ROWS, _auto_choice, _auto_parts, _launch_auto, _refined
+from feather_ops.scaled_mm import _TAIL_MAX_ROWS, _auto_choice, _auto_parts, _auto_plan, _launch_auto, _refined
 
 FP16, BF16 = torch.float16, torch.bfloat16
 
@@ -52,6 +52,25 @@ def test_parts_cover_the_rows_once():
 def test_empty_sides_are_one_launch(m, n, k, dtype):
     """The op itself answers them: an empty result, or its refusal of K."""
     assert _auto_parts(m, n, k, dtype) == (((m, *_auto_choice(m, n, k, dtype)[:2]),), _auto_choice(m, n, k, dtype)[2])
+
+
+@pytest.mark.parametrize("m,n,k", SPLIT + [(16, 1000, 2560), (77, 5120, 2560), (4096, 4096, 4096), (40, 5120, 12288)])
+def test_traced_sizes(m, n, k):
+    """torch.jit.trace passes sizes as tensors: the same plan, in plain numbers."""
+    for dtype in (FP16, BF16):
+        plan = _auto_plan(torch.tensor(m), torch.tensor(n), torch.tensor(k), dtype)
+        assert repr(plan) == repr(_auto_plan(m, n, k, dtype))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [SPLIT[1], SPLIT[5], (16, 1000, 2560)])
+def test_jit_trace(m, n, k):
+    import feather_ops
+
+    a, b, scale, bias = _inputs(m, n, k, BF16, True)
+    want = feather_ops.scaled_mm_hip(a, b, scale, bias, BF16)
+    traced = torch.jit.trace(lambda x: feather_ops.scaled_mm_hip(x, b, scale, bias, BF16), (a,), check_trace=False)
+    assert torch.equal(traced(a), want)
 
 
 def _inputs(m, n, k, dtype, column):

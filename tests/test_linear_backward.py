@@ -47,6 +47,16 @@ def test_plans_pass_the_librarys_check(m, n, k):
     assert lib.feather_linear_backward_split_bytes(m, n + 4, k, False, *tile, 1) == -1
 
 
+def test_only_small_layers_and_big_buffers_have_no_plan():
+    rng = random.Random(1)
+    for _ in range(4000):
+        m, n, k = int(2 ** rng.uniform(0, 15)), 8 * int(2 ** rng.uniform(0, 11)), 16 * int(2 ** rng.uniform(0, 10))
+        for column in (False, True):
+            depth = 48 * -(-n // 16) if column else n + n % 16
+            fits = max(2 * m * max(n, k, depth), -(-depth // 128) * 128 * k) < 1 << 31
+            assert (lb.backward_plan(m, n, k, column) is not None) == (m * n * k >= 1 << 22 and fits), (m, n, k, column)
+
+
 def test_plan_refuses_buffers_past_2_gib():
     assert lb.backward_plan(65536, 8192, 4096, True) is None      # the split gradient: 3.2 GB
     assert lb.backward_plan(65536, 8192, 4096, False) is not None
